@@ -25,8 +25,18 @@ __global__ __launch_bounds__(256) void k_reduce(ReduceArgs a) {
     const unsigned c = (unsigned)(r / a.Ng);
     const float *p = a.part + ((((unsigned long long)c * a.Ng + g) * a.G) * a.Q + q) * a.N + jo;
     const unsigned long long step = (unsigned long long)a.Q * a.N;
+    // partials in order, eight loads in flight: a launch of few outputs is
+    // bound by the chain of loads (64 partials of 65536 outputs: 42 to 12 us)
     float sum = 0.0f;
-    for (unsigned ch = 0; ch < a.G; ++ch) sum += p[ch * step];
+    unsigned ch = 0;
+    for (; ch + 8 <= a.G; ch += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = p[(ch + u) * step];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) sum += v[u];
+    }
+    for (; ch < a.G; ++ch) sum += p[ch * step];
     float *o = a.acc + (((unsigned long long)g * a.Q + q) * a.Nc + c) * a.N + jo;
     const float val = sum * a.scale;
     *o = a.first ? val : (*o + val);

@@ -10,6 +10,18 @@ namespace rsk {
 constexpr int kTwLog = 12;            // master twiddle table: W_4096^m
 constexpr int kTwN = 1 << kTwLog;     // also the largest single-pass FFT
 
+// Behind the W_4096 table: the constants of the transforms that begin on the
+// matrix cores (dft_hybrid.h).  First the FP16 operands of the 32-point DFT
+// matrix (kHybOperands float2 of memory), then for M = 2, 4, .. 32 the
+// hyb_ntw(M) butterfly factors (tan, cos) of each of 64 lanes.
+constexpr int kHybOperands = 2 * 4 * 2 * 64 * 16 / 8;
+// factors of in-lane sub-transforms below size m: one for sizes 2 and 4,
+// m / 4 above
+constexpr int dit_off(int m) { return m <= 2 ? 0 : dit_off(m / 2) + (m / 2 <= 4 ? 1 : m / 8); }
+constexpr int hyb_ntw(int M) { return M == 32 ? 9 : (M <= 2 ? 1 : dit_off(M) + (M >= 8 ? M / 4 : 1)); }
+constexpr int hyb_tw_off(int M) { return M <= 2 ? 0 : hyb_tw_off(M / 2) + 64 * hyb_ntw(M / 2); }
+constexpr int kTwTotal = kTwN + kHybOperands + hyb_tw_off(64);   // float2 of the device table
+
 // Fused small-N path (N <= 4096): unpack -> FFT -> detect -> integrate a
 // chunk of `chunk` spectra.  Workgroup b covers channel b / bpc and either
 // groups [gpw*(b % bpc), +gpw) whole, or chunk (b % bpc) % G of group
@@ -32,7 +44,7 @@ struct SmallArgs {
   int first;                      // direct: overwrite (1) or accumulate (0)
   float *acc;                     // [Nds][Q][Nc][N], FFT-shifted
   float *part;                    // [Nc][Ng][G][Q][N] unscaled, FFT-shifted
-  const float2 *tw;               // W_4096^m, m < 4096
+  const float2 *tw;               // W_4096^m, m < 4096, and behind it kTwTotal's rest
   // transform length: the kernel's N, or for a product whose length is not
   // a power of two (Bluestein, N >= 2 nt - 1) nt with its tables
   unsigned nt;
@@ -75,7 +87,7 @@ struct FsArgs {
   float2 *work;                   // Y for the chunk
   float *acc;                     // host layout [Nds][Q][Nc][N]
   float *acc_int;                 // internal accumulator (Nis > 1)
-  const float2 *tw;               // W_4096^m
+  const float2 *tw;               // W_4096^m, and behind it kTwTotal's rest
   const float2 *twf;              // W_N^r, r < N1 (N1 <= 4096)
   // Y holds ynb buffers' spectra per channel ([cl][slot * Nss + sp]); pass A
   // writes this launch's nbat buffers to slots yb0 .., pass B reads slots
@@ -123,6 +135,14 @@ int launch_fs_b(int np, int pmode, const FsArgs &a, hipStream_t s);
 // The ns runs' sums of a split pass B, in run order, then pass B's own
 // finish (scale, internal accumulator, shifted output) for a.mode.
 int launch_fs_b_reduce(int pmode, const FsArgs &a, hipStream_t s);
+// The fused small kernel with its first 32 points on the matrix cores (N = 64
+// .. 1024, a group's spectra in this buffer a multiple of 1024 / N).  solo:
+// each wavefront integrates gpw whole groups, bpc wavefronts per channel,
+// nblocks workgroups of 4 wavefronts; otherwise one workgroup of 4 or 8
+// wavefronts (waves) per (channel, group, chunk).
+int small_h_ok(int n, unsigned na_buf);
+int launch_small_h(int n, int nbps, int np, int pmode, const SmallArgs &a, unsigned nblocks, int solo,
+                   int waves, hipStream_t s);
 // Matrix-core fused small kernel (N = 1024, two pols): one wavefront per
 // (channel, group, chunk) item, items = Nc * Ng * G, gpw must be 1.
 int small_mfma_ok(int n, int np);

@@ -67,6 +67,10 @@ struct ProdPlan {
   int m_ok;
   unsigned m_chunk, m_G;
   int m_unsplit;           // int8 samples, long enough integration: unsplit FP16 operands allowed
+  // small kernel with its first stage on the matrix cores (h_ok: it takes
+  // the vector kernel's place); h_solo: whole groups per wavefront
+  int h_ok, h_solo, h_waves;
+  unsigned h_chunk, h_G, h_gpw, h_bpc;
   // four-step path
   unsigned N1, N2;
   unsigned fs_chunk;       // channels per pass A/B launch pair (one buffer)
@@ -202,6 +206,49 @@ std::vector<float2> twiddles(unsigned long long n, unsigned long long cnt, unsig
   return t;
 }
 
+// Constants of the transforms that begin on the matrix cores, laid out behind
+// the W_4096 table as kernels.h states, from FP64.
+void hybrid_tables(std::vector<float2> &t) {
+  const size_t base = t.size();
+  t.resize(rsk::kTwTotal);
+  _Float16 *b = reinterpret_cast<_Float16 *>(t.data() + base);
+  // operand [re/im output][K-block][hi/lo][lane][8]: K element 2 i + part of
+  // lane (col, h) is complex row 8 kb + 4 h + i of the 32-point DFT matrix
+  for (int o = 0; o < 2; ++o)
+    for (int kb = 0; kb < 4; ++kb)
+      for (int lane = 0; lane < 64; ++lane)
+        for (int i = 0; i < 4; ++i) {
+          const int row = 8 * kb + 4 * (lane >> 5) + i, col = lane & 31;
+          const double ang = -2.0 * M_PI * (double)((row * col) & 31) / 32.0;
+          const double re = cos(ang), im = sin(ang);
+          // real output: re(x) re - im(x) im; imaginary output: re(x) im + im(x) re
+          const double v[2] = {o == 0 ? re : im, o == 0 ? -im : re};
+          for (int part = 0; part < 2; ++part) {
+            const _Float16 hi = (_Float16)(float)v[part];
+            const _Float16 lo = (_Float16)(float)(v[part] - (double)(float)hi);
+            _Float16 *at = b + ((size_t)((o * 4 + kb) * 2) * 64 + lane) * 8 + 2 * i + part;
+            at[0] = hi;
+            at[64 * 8] = lo;
+          }
+        }
+  float2 *f = t.data() + base + rsk::kHybOperands;
+  auto put = [&](int M, int k, int lane, int m, int x) {
+    const double ang = -2.0 * M_PI * (double)x / (32.0 * m);
+    f[rsk::hyb_tw_off(M) + 64 * k + lane] = make_float2((float)(sin(ang) / cos(ang)), (float)cos(ang));
+  };
+  for (int lane = 0; lane < 64; ++lane) {
+    const int c = lane & 31, h = lane >> 5;
+    for (int M = 2; M <= 16; M *= 2)
+      for (int m = 2; m <= M; m *= 2)
+        for (int k = 0; k < (m >= 8 ? m / 4 : 1); ++k) put(M, rsk::dit_off(m) + k, lane, m, c + 32 * k);
+    put(32, 0, lane, 2, c);
+    put(32, 1, lane, 4, c);
+    put(32, 2, lane, 8, c + 32 * h);
+    for (int k = 0; k < 2; ++k) put(32, 3 + k, lane, 16, c + 32 * (h + 2 * k));
+    for (int k = 0; k < 4; ++k) put(32, 5 + k, lane, 32, c + 32 * (h + 2 * k));
+  }
+}
+
 }  // namespace
 
 struct rsd_ctx {
@@ -306,10 +353,14 @@ static void plan_small(rsd_ctx *d, ProdPlan &pp) {
   pp.na_buf = pp.p.Na < pp.p.Nss ? pp.p.Na : pp.p.Nss;
   pp.Ng = pp.p.Nss / pp.na_buf;
   pp.chunk = pp.na_buf;
+  const unsigned n = pp.bs ? pp.bs_m : pp.p.Nt;
   // Split long groups over workgroups until the launch fills the device
   // (by default about 2048 workgroups for 256 CUs), keeping >= one spectrum
-  // per slot.
-  const unsigned long long target = pp.t_target;
+  // per slot.  From 2048 points a workgroup's one or two slots hold a CU's
+  // registers for two workgroups: 512 of them fill it, and more only write
+  // partial sums (4096 points, Stokes, 64 MiB in dumps of 4 spectra: 67
+  // against 141 us).
+  const unsigned long long target = n >= 2048 ? pp.t_target / 4 : pp.t_target;
   while ((unsigned long long)Nc * pp.Ng * (pp.na_buf / pp.chunk) < target && pp.chunk % 2 == 0 &&
          pp.chunk / 2 >= slots)
     pp.chunk /= 2;
@@ -326,6 +377,13 @@ static void plan_small(rsd_ctx *d, ProdPlan &pp) {
   if (pp.G == 1) {
     unsigned spg = 1;
     while (spg < pp.chunk && spg < kMaxSpg) spg <<= 1;
+    // more slots for a long group where that makes too few wavefronts (8
+    // points in dumps of 1024 spectra, 64 MiB: 17 against 47 us; shorter
+    // dumps fill the device as they are and lose by it, 16 against 22)
+    const unsigned long long fill = 8192ull * 64 / (unsigned)rsk::small_wg((int)n);
+    while (spg < slots && pp.chunk >= 8 * spg &&
+           (unsigned long long)Nc * ((pp.Ng + slots / spg - 1) / (slots / spg)) < fill)
+      spg <<= 1;
     if (spg < slots) {
       pp.spg = spg;
       pp.gpw = slots / spg;
@@ -355,9 +413,56 @@ static void plan_small_mfma(rsd_ctx *d, ProdPlan &pp) {
   pp.m_G = pp.na_buf / pp.m_chunk;
 }
 
+// Plan of the small kernel whose first 32 points run on the matrix cores
+// (k_small_h.hip).  Where the channels' groups alone make kHybSoloWaves
+// wavefronts, each wavefront integrates whole groups; otherwise the groups
+// are halved into chunks until t_target / 4 workgroups are busy (default 512,
+// two per CU: 1024 read 64 MiB no faster and wrote twice the partial sums),
+// each of a chunk's 4 wavefronts keeping a unit of 1024 samples.
+constexpr unsigned kHybSoloWaves = 2048;
+static void plan_small_h(rsd_ctx *d, ProdPlan &pp) {
+  // int16 power of 64 and 256 points is near the memory's rate on the vector
+  // units (one LDS exchange): 55 and 68 against 69 and 82 us per 256 MiB here
+  pp.h_ok = !pp.bs && rsk::small_h_ok((int)pp.p.Nt, pp.na_buf) &&
+            !(d->cfg.Nbps == 16 && d->cfg.Np == 2 && pp.p.npolout == 1 &&
+              (pp.p.Nt == 64 || pp.p.Nt == 256));
+  if (!pp.h_ok) return;
+  const unsigned S = 1024u / pp.p.Nt, Nc = d->cfg.Nc;
+  const unsigned upg = pp.na_buf / S;          // units per group
+  pp.h_chunk = pp.na_buf;
+  pp.h_G = 1;
+  pp.h_gpw = 1;
+  pp.h_bpc = 1;
+  pp.h_waves = 4;
+  const unsigned long long groups = (unsigned long long)Nc * pp.Ng;
+  pp.h_solo = groups >= kHybSoloWaves || upg < 4;
+  if (pp.h_solo) {
+    // at most 8 wavefronts per SIMD's two slots, so that the last round is short
+    unsigned gpw = (unsigned)(groups / (8ull * kHybSoloWaves));
+    if (gpw < 1) gpw = 1;
+    if (gpw > pp.Ng) gpw = pp.Ng;
+    pp.h_gpw = gpw;
+    pp.h_bpc = (pp.Ng + gpw - 1) / gpw;
+    return;
+  }
+  while (groups * pp.h_G < pp.t_target / 4 && pp.h_chunk % (2 * S) == 0 && pp.h_chunk / (2 * S) >= 4) {
+    pp.h_chunk /= 2;
+    pp.h_G *= 2;
+  }
+  // two chunks fit one workgroup of 8 wavefronts, which saves the partial
+  // sums and the launch that adds them (longer serial chains do not pay: 16
+  // units by 8 wavefronts 11.0 us, by 16 and k_reduce 9.9)
+  if (pp.h_G == 2) {
+    pp.h_waves = 8;
+    pp.h_chunk = pp.na_buf;
+    pp.h_G = 1;
+  }
+}
+
 static size_t part_need(const rsd_ctx *d, const ProdPlan &pp) {
   if (!pp.small) return 0;
-  size_t n = pp.direct ? 0 : (size_t)d->cfg.Nc * pp.Ng * pp.G * pp.Q * pp.p.Nt;
+  const unsigned G = pp.h_ok ? pp.h_G : (pp.direct ? 1u : pp.G);
+  size_t n = G > 1 ? (size_t)d->cfg.Nc * pp.Ng * G * pp.Q * pp.p.Nt : 0;
   if (pp.m_ok && pp.m_G > 1) {
     const size_t m = (size_t)d->cfg.Nc * pp.Ng * pp.m_G * pp.Q * pp.p.Nt;
     if (m > n) n = m;
@@ -531,6 +636,7 @@ static size_t plan_product(rsd_ctx *d, ProdPlan &pp) {
   if (pp.small) {
     plan_small(d, pp);
     plan_small_mfma(d, pp);
+    plan_small_h(d, pp);
   } else {
     const unsigned L = ilog2u(N);
     pp.N1 = 1u << ((L + 1) / 2);
@@ -646,7 +752,7 @@ static int plan_all(const rsd_config *cfg, rsd_ctx *d) {
 // Device bytes the plan allocates.
 static size_t plan_bytes(const rsd_ctx *d) {
   size_t b = d->in_bytes + (d->cfg.expand4 ? (size_t)(d->chan_block_bytes / 2) * d->cfg.Nc : 0);
-  b += (size_t)rsk::kTwN * sizeof(float2) + (d->cfg.ics ? d->cfg.Nant * sizeof(float) : 0);
+  b += (size_t)rsk::kTwTotal * sizeof(float2) + (d->cfg.ics ? d->cfg.Nant * sizeof(float) : 0);
   size_t held = 0;
   for (unsigned i = 0; i < d->cfg.No; ++i) {
     const ProdPlan &pp = d->pp[i];
@@ -680,7 +786,12 @@ static int create_impl(const rsd_config *cfg, rsd_ctx *d) {
     return 1;
   // master twiddle table W_4096^m
   {
-    std::vector<float2> t = twiddles(rsk::kTwN, rsk::kTwN, 1);
+    // the same for every context: computed once per process
+    static const std::vector<float2> t = [] {
+      std::vector<float2> v = twiddles(rsk::kTwN, rsk::kTwN, 1);
+      hybrid_tables(v);
+      return v;
+    }();
     RSD_CHECK(hipMalloc(&d->d_tw, t.size() * sizeof(float2)));
     RSD_CHECK(hipMemcpy(d->d_tw, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice));
   }
@@ -866,6 +977,19 @@ static int run_small(rsd_ctx *d, int i, const uint8_t *in, float isign, float ga
                                  (unsigned)items, s))
         return 1;
     }
+  } else if (pp.h_ok) {
+    a.chunk = pp.h_chunk;
+    a.G = pp.h_G;
+    a.gpw = pp.h_gpw;
+    a.bpc = pp.h_bpc;
+    a.direct = pp.h_G == 1;
+    const unsigned long long nb = pp.h_solo ? ((unsigned long long)pp.h_bpc * c.Nc + 3) / 4
+                                            : (unsigned long long)c.Nc * pp.Ng * pp.h_G;
+    if (nb > 0x7fffffffull) return 1;
+    ProfScope ps(d, i, "k_small", pp.p.Nt, s);
+    if (rsk::launch_small_h((int)pp.p.Nt, (int)c.Nbps, (int)c.Np, pp.p.npolout, a, (unsigned)nb,
+                            pp.h_solo, pp.h_waves, s))
+      return 1;
   } else {
     const unsigned long long nb = (unsigned long long)pp.bpc * c.Nc;
     if (nb > 0x7fffffffull) return 1;
@@ -1219,6 +1343,7 @@ static std::vector<Tunables> tune_cands(const rsd_ctx *d, const ProdPlan &pp) {
 
 // The launch plan the current tunables produce, for skipping duplicates.
 static std::vector<unsigned long long> plan_key(const ProdPlan &pp) {
+  if (pp.small && pp.h_ok) return {pp.h_chunk, pp.h_gpw, pp.m_chunk};
   if (pp.small) return {pp.chunk, pp.G, pp.spg, pp.gpw, pp.m_chunk};
   return {pp.fs_chunk, pp.fs_bmax};
 }
