@@ -227,6 +227,18 @@ def lib():
     return _lib
 
 
+class DevicePointer(int):
+    """A device address (an int) that keeps the context owning the memory
+    alive: an array made from it (through __cuda_array_interface__, which the
+    consumer holds on to) must not outlive the buffers, which are freed when
+    the Spectrometer is collected."""
+
+    def __new__(cls, value, owner):
+        p = super().__new__(cls, value)
+        p.owner = owner
+        return p
+
+
 class Spectrometer:
     """Thin convenience owner of one ``rawspec_context``.
 
@@ -321,13 +333,13 @@ class Spectrometer:
         return lib().rawspec_amd_set_device_output(C.byref(self.ctx), 1 if enable else 0)
 
     def device_input(self) -> int:
-        return lib().rawspec_amd_device_input(C.byref(self.ctx)) or 0
+        return DevicePointer(lib().rawspec_amd_device_input(C.byref(self.ctx)) or 0, self)
 
     def device_input_size(self) -> int:
         return lib().rawspec_amd_device_input_size(C.byref(self.ctx))
 
     def device_pwrbuf(self, i) -> int:
-        return lib().rawspec_amd_device_pwrbuf(C.byref(self.ctx), i) or 0
+        return DevicePointer(lib().rawspec_amd_device_pwrbuf(C.byref(self.ctx), i) or 0, self)
 
     def stream(self) -> int:
         return lib().rawspec_amd_stream(C.byref(self.ctx)) or 0
@@ -390,6 +402,12 @@ class Spectrometer:
         return lib().rawspec_wait_for_completion(C.byref(self.ctx))
 
     # -- numpy views -----------------------------------------------------
+    # Each view holds on to the context, whose buffers it shows.
+    def _view(self, ctype, n, ptr) -> np.ndarray:
+        a = (ctype * n).from_address(ptr)
+        a.owner = self
+        return np.ctypeslib.as_array(a)
+
     @property
     def blocsize(self) -> int:
         c = self.ctx
@@ -400,17 +418,17 @@ class Spectrometer:
         ptr = self.ctx.h_blkbufs[i]
         if not ptr:
             raise RuntimeError(f"host block {i} is not allocated")
-        return np.ctypeslib.as_array((C.c_uint8 * self.blocsize).from_address(ptr))
+        return self._view(C.c_uint8, self.blocsize, ptr)
 
     def pwrbuf(self, i) -> np.ndarray:
         n = self.ctx.h_pwrbuf_size[i] // 4
         ptr = C.cast(self.ctx.h_pwrbuf[i], C.c_void_p).value
-        return np.ctypeslib.as_array((C.c_float * n).from_address(ptr))
+        return self._view(C.c_float, n, ptr)
 
     def icsbuf(self, i) -> np.ndarray:
         n = self.ctx.h_pwrbuf_size[i] // 4 // self.ctx.Nant
         ptr = C.cast(self.ctx.h_icsbuf[i], C.c_void_p).value
-        return np.ctypeslib.as_array((C.c_float * n).from_address(ptr))
+        return self._view(C.c_float, n, ptr)
 
     def close(self):
         self.cleanup()
