@@ -29,11 +29,11 @@ ARCH = os.environ.get("RAWSPEC_AMD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CC = os.environ.get("CC", "gcc")
 
-HIP_SOURCES = ["rsd_runtime.hip", "k_small.hip", "k_small_h.hip", "k_fourstep.hip", "k_mfma.hip", "k_misc.hip"]
+HIP_SOURCES = ["rsd_runtime.hip", "k_small.hip", "k_small_h.hip", "k_fourstep.hip", "k_fs_a_h.hip", "k_mfma.hip", "k_misc.hip"]
 C_SOURCES = ["rawspec_api.c", "raw_header.c", "fb_header.c"]
 
 HIP_FLAGS = [
-    f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17",
+    f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++20",
     # packed FP32 instructions stay disabled for all device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument",

@@ -48,17 +48,21 @@ struct Dft32K {
 
 // The constants come from a table the host computes in 64 bits (behind the
 // W_4096 table, kernels.h): the operands, then stage 2's factors of every M.
-__device__ __forceinline__ void dft32_consts(Dft32K &k, const float2 *tw4096, int wg) {
+// sgn = 0x80000000 negates the rows that meet imaginary parts: the transform
+// of the conjugated samples.
+__device__ __forceinline__ void dft32_consts(Dft32K &k, const float2 *tw4096, int wg, unsigned int sgn) {
   const uint4 *src = reinterpret_cast<const uint4 *>(tw4096 + kTwN);
   uint4 *dst = reinterpret_cast<uint4 *>(&k);
-  for (int e = threadIdx.x; e < (int)(sizeof(Dft32K) / 16); e += wg) dst[e] = src[e];
+  for (int e = threadIdx.x; e < (int)(sizeof(Dft32K) / 16); e += wg) {
+    const uint4 v = src[e];
+    dst[e] = make_uint4(v.x ^ sgn, v.y ^ sgn, v.z ^ sgn, v.w ^ sgn);
+  }
 }
 
 // ---- samples -> FP16 operands ----------------------------------------------
 // One sample word to the (re, im) FP16 pair of each pol (HybIn::hi) and, for
-// int16, the pair of fractions (lo).  sgn is 0, or 0x80000000 to conjugate
-// (int8: exact sign flip of the imaginary half; int16: of both parts).  The
-// SNORM clamp of the most negative code is applied.
+// int16, the pair of fractions (lo).  The SNORM clamp of the most negative code
+// is applied.
 template <int NBPS, int NP>
 struct HybIn;
 template <int NP>
@@ -67,8 +71,8 @@ struct HybIn<8, NP> {
   static constexpr float SCALE = 1.0f;         // Z scale: samples as they are
   using word = typename Sample<8, NP>::word;
   template <int P>
-  __device__ __forceinline__ static void pair(word w, unsigned int &hi, unsigned int &, unsigned int sgn) {
-    hi = i8_pair_f16<P>((unsigned int)w ^ 0x80808080u) ^ sgn;
+  __device__ __forceinline__ static void pair(word w, unsigned int &hi, unsigned int &) {
+    hi = i8_pair_f16<P>((unsigned int)w ^ 0x80808080u);
   }
 };
 template <int NP>
@@ -78,7 +82,7 @@ struct HybIn<16, NP> {
   using word = typename Sample<16, NP>::word;
   typedef short s2v __attribute__((ext_vector_type(2)));
   template <int P>
-  __device__ __forceinline__ static void pair(word w, unsigned int &hi, unsigned int &lo, unsigned int sgn) {
+  __device__ __forceinline__ static void pair(word w, unsigned int &hi, unsigned int &lo) {
     unsigned int v;
     if constexpr (NP == 2) v = P == 0 ? w.x : w.y;
     else v = w;
@@ -90,8 +94,8 @@ struct HybIn<16, NP> {
     // low bytes under exponent byte 0x44: 4 + lo / 256
     const h2v l = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x44444444u, v, 0x04020400u)) -
                   (h2v){(_Float16)4.0f, (_Float16)4.0f};
-    hi = __builtin_bit_cast(unsigned int, h) ^ sgn;
-    lo = __builtin_bit_cast(unsigned int, l) ^ sgn;
+    hi = __builtin_bit_cast(unsigned int, h);
+    lo = __builtin_bit_cast(unsigned int, l);
   }
 };
 

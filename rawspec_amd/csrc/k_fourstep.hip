@@ -1,4 +1,6 @@
-// k_fourstep.hip -- spectrometer kernels for FFT lengths 8192 .. 2^24.
+// k_fourstep.hip -- spectrometer kernels for FFT lengths 8192 .. 2^24 (pass A:
+// from 2^18 points with the 24-bit intermediate, else 2^19; k_fs_a_h.hip has the
+// shorter ones).
 //
 // Bailey's four-step decomposition N = N1*N2 (n = n1 + N1*n2,
 // k = k2 + N2*k1):
@@ -295,6 +297,12 @@ int fs_tile_b(int n1) { return (int)(wg_team(n1) / (n1 / elems_fs(n1))); }
 template <int N2, int R1, int NBPS>
 static int go_a_r(int np, const FsArgs &a, unsigned nb, hipStream_t s) {
   constexpr int WGT = wg_team(N2);
+  // 2^18 points: only the 24-bit intermediate comes here (k_fs_a_h.hip)
+  if constexpr (N2 == 512 && R1 == 1) {
+    if (np != 2 || !a.y24) return 2;
+    hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 2, true>), dim3(nb), dim3(WGT), 0, s, a);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
+  }
   if (np == 2 && a.y24) hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 2, true>), dim3(nb), dim3(WGT), 0, s, a);
   else if (np == 2) hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 2, false>), dim3(nb), dim3(WGT), 0, s, a);
   else hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 1, false>), dim3(nb), dim3(WGT), 0, s, a);
@@ -313,9 +321,6 @@ static int go_a(int np, const FsArgs &a, unsigned nb, hipStream_t s) {
 template <int NBPS>
 static int go_a_n(int np, const FsArgs &a, unsigned nb, hipStream_t s) {
   switch (a.N2) {
-    case 64: return go_a<64, NBPS>(np, a, nb, s);
-    case 128: return go_a<128, NBPS>(np, a, nb, s);
-    case 256: return go_a<256, NBPS>(np, a, nb, s);
     case 512: return go_a<512, NBPS>(np, a, nb, s);
     case 1024: return go_a<1024, NBPS>(np, a, nb, s);
     case 2048: return go_a<2048, NBPS>(np, a, nb, s);

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(64 * WAVES, PMODE == 1 && !(NBPS == 16 && NP == 2 &
     nu = (unsigned)wv < cu ? (cu - wv + WAVES - 1) / WAVES : 0;
   }
 
-  dft32_consts(K, a.tw, 64 * WAVES);
+  dft32_consts(K, a.tw, 64 * WAVES, 0u);
   float2 tg[hyb_ntw(M)];
   hyb_tw<M>(tg, a.tw, lane);
   __syncthreads();
@@ -131,8 +131,8 @@ __global__ __launch_bounds__(64 * WAVES, PMODE == 1 && !(NBPS == 16 && NP == 2 &
         unsigned int hi, lo = 0;
         if constexpr (NBPS == 16 && NP == 2)
           HybIn<16, 1>::template pair<0>(reinterpret_cast<const unsigned int *>(tr + E + PAD * (E >> 6))[p],
-                                         hi, lo, 0u);
-        else In::template pair<p>(tr[E + PAD * (E >> 6)], hi, lo, 0u);
+                                         hi, lo);
+        else In::template pair<p>(tr[E + PAD * (E >> 6)], hi, lo);
         frag_set(f, e, hi, lo);
       }
     };

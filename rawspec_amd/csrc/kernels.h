@@ -131,6 +131,10 @@ int fs_tile_b(int n1);          // k2 values per pass-B workgroup
 int launch_small(int n, int nbps, int np, int pmode, const SmallArgs &a,
                  unsigned nblocks, hipStream_t s);
 int launch_fs_a(int nbps, int np, const FsArgs &a, hipStream_t s);
+// Pass A with its first 32 points on the matrix cores (N1 = 128 .. 512): the
+// same contract and layout; a.grid_a workgroups loop over the tiles.
+int fs_a_h_ok(int n1, int n2, int y24);
+int launch_fs_a_h(int nbps, int np, const FsArgs &a, hipStream_t s);
 int launch_fs_b(int np, int pmode, const FsArgs &a, hipStream_t s);
 // The ns runs' sums of a split pass B, in run order, then pass B's own
 // finish (scale, internal accumulator, shifted output) for a.mode.

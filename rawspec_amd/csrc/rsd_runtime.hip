@@ -1127,6 +1127,12 @@ static void fs_args(rsd_ctx *d, ProdPlan &pp, rsk::FsArgs &a, float isign, float
 #define RSD_FSA_MFMA_WG_PER_CU 2
 #endif
 
+// Workgroups per CU of the pass A that begins on the matrix cores (two are
+// resident), each wavefront looping over its share of the tiles.
+#ifndef RSD_FSA_H_WG_PER_CU
+#define RSD_FSA_H_WG_PER_CU 8
+#endif
+
 static int launch_pass_a(rsd_ctx *d, int i, rsk::FsArgs a, hipStream_t s) {
   ProdPlan &pp = d->pp[i];
   if (pp.fs_amfma) {
@@ -1135,6 +1141,10 @@ static int launch_pass_a(rsd_ctx *d, int i, rsk::FsArgs a, hipStream_t s) {
     return rsk::launch_fs_a_mfma((int)d->cfg.Nbps, (int)d->cfg.Np, a, s);
   }
   ProfScope ps(d, i, "k_fs_a", pp.p.Nt, s);
+  if (rsk::fs_a_h_ok((int)pp.N1, (int)pp.N2, a.y24)) {
+    a.grid_a = d->cus * RSD_FSA_H_WG_PER_CU;
+    return rsk::launch_fs_a_h((int)d->cfg.Nbps, (int)d->cfg.Np, a, s);
+  }
   return rsk::launch_fs_a((int)d->cfg.Nbps, (int)d->cfg.Np, a, s);
 }
 

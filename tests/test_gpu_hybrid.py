@@ -7,12 +7,14 @@ workgroup, integrations over buffers) for both sample widths, one and two
 pols, all modes, both directions.
 
 The bar is the FP32 engine's: 1e-5 of the total power of the bin or of the
-channel's mean, whichever is larger."""
+channel's mean, whichever is larger (four-step products: the rule of
+spectro_cases.check_results, five times a single-precision reference's
+error where that is more)."""
 import numpy as np
 import pytest
 
 import oracle as O
-from tests.spectro_cases import PLAIN_TOL, rel_err
+from tests.spectro_cases import PLAIN_TOL, check_results, rel_err, run_device_case
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +89,19 @@ def test_two_chunks_share_a_workgroup():
     for mode, bits in ((-4, 8), (1, 16)):
         assert run(Nc=32, Ntpb=1024 * 64, Nts=[1024], Nas=[8], Np=2, bits=bits, pols=[mode], fwd=True,
                    conj=0) <= PLAIN_TOL
+
+
+@pytest.mark.parametrize("bits", [8, 16])
+@pytest.mark.parametrize("np_", [1, 2])
+@pytest.mark.parametrize("lg", [13, 14, 15, 16, 17, 18])
+def test_fourstep_first_pass(lg, np_, bits):
+    nt = 1 << lg
+    for level in (0, 1):
+        fwd = 1 if (lg + bits // 8 + level) % 2 else -1
+        modes = [-4, 4] if np_ == 2 else [1, 1]
+        kw = dict(Nc=3, Ntpb=2 * nt, Nts=[nt, nt], Nas=[1, 6], Np=np_, Nbps=bits, Npolout=modes, nbuf=3,
+                  batches=[1, 2], fft_dir=fwd, conj=level, seed=lg, sigma=8.0 if bits == 8 else 900.0,
+                  tone=(1, 20.0, 300.0, 1024.0), mfma=level)
+        print(f"case: {kw}", flush=True)
+        res, cfg = run_device_case(**kw)
+        check_results(res, cfg, tol_by_product={0: 1e-3, 1: 1e-3} if level else None)
