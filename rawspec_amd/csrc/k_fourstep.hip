@@ -408,8 +408,18 @@ __global__ __launch_bounds__(256) void k_fs_b_reduce(FsArgs a, unsigned Q, unsig
     r /= tiles;
     const unsigned cl = (unsigned)(r % a.nch);
     const unsigned g = (unsigned)(r / a.nch);
+    // runs in order, eight loads in flight (a chain of 64 single loads took
+    // 30 us, as long as pass B)
     float sum = 0.0f;
-    for (unsigned run = 0; run < a.ns; ++run) sum += load_acc(a.partb + run * total + idx);
+    unsigned run = 0;
+    for (; run + 8 <= a.ns; run += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = load_acc(a.partb + (run + u) * total + idx);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) sum += v[u];
+    }
+    for (; run < a.ns; ++run) sum += load_acc(a.partb + run * total + idx);
     float v = sum * a.scale;
     const unsigned c = a.c0 + cl;
     float *ie = a.acc_int + ((((unsigned long long)g * a.Nc + c) * tiles + tile) * Q + q) * N1 * TB +

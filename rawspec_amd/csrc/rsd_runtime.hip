@@ -129,11 +129,8 @@ constexpr size_t kHoldBytes = (size_t)RSD_HOLD_MB << 20;
 // are fewer; the fewest spectra a run integrates; the CU count the planner
 // sizes the runs' partial sums for (launches use the device's own count,
 // capped by what was allocated).
-#ifndef RSD_FSB_MIN_RUN
-#define RSD_FSB_MIN_RUN 8
-#endif
 constexpr unsigned kFsbWgPerCu = 4;
-constexpr unsigned kFsbMinRun = RSD_FSB_MIN_RUN;
+constexpr unsigned kFsbMinRun = 1;
 constexpr unsigned kPlanCus = 256;
 
 bool is_pow2(unsigned n) { return n && !(n & (n - 1)); }
@@ -604,7 +601,10 @@ static unsigned fsb_runs(const ProdPlan &pp, unsigned cus, unsigned Nc, unsigned
   const unsigned long long target = (unsigned long long)cus * kFsbWgPerCu;
   if (base == 0 || base >= target) return 1;
   unsigned long long ns = (target + base - 1) / base;
-  const unsigned maxr = na_buf / kFsbMinRun;
+  // groups of two or three spectra save less than the runs' launch costs; from
+  // four on a spectrum per run is best (2^16 points, 2 channels, 4 spectra: 52
+  // us whole, 38 in runs of two, 28 in runs of one)
+  const unsigned maxr = na_buf < 4 ? 1 : na_buf / kFsbMinRun;
   if (ns > maxr) ns = maxr;
   return ns < 1 ? 1u : (unsigned)ns;
 }
