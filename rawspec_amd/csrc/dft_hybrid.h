@@ -143,43 +143,6 @@ __device__ __forceinline__ void dft32_mfma(const HybFrag<PARTS> (&f)[NP], const 
 }
 
 // ---- stage 2 -----------------------------------------------------------------
-// E +- w O with w = g (1 + i t), or w = -i g (1 + i t) when ROT.
-template <bool ROT>
-__device__ __forceinline__ void bfly(const float2 e, const float2 o, const float2 tg, float2 &lo, float2 &hi) {
-  const float u = fmaf(-tg.x, o.y, o.x), v = fmaf(tg.x, o.x, o.y);
-  if constexpr (!ROT) {
-    lo = make_float2(fmaf(tg.y, u, e.x), fmaf(tg.y, v, e.y));
-    hi = make_float2(fmaf(-tg.y, u, e.x), fmaf(-tg.y, v, e.y));
-  } else {
-    lo = make_float2(fmaf(tg.y, v, e.x), fmaf(-tg.y, u, e.y));
-    hi = make_float2(fmaf(-tg.y, v, e.x), fmaf(tg.y, u, e.y));
-  }
-}
-
-// In-lane decimation in time of M points in natural order, factors tg[dit_off(m) + k].
-template <int M>
-struct MDit {
-  template <int NT>
-  __device__ __forceinline__ static void run(float2 (&x)[M], const float2 (&tg)[NT]) {
-    float2 e[M / 2], o[M / 2];
-#pragma unroll
-    for (int k = 0; k < M / 2; ++k) { e[k] = x[2 * k]; o[k] = x[2 * k + 1]; }
-    MDit<M / 2>::run(e, tg);
-    MDit<M / 2>::run(o, tg);
-    constexpr int G = M >= 8 ? M / 4 : 1, OFF = dit_off(M);
-#pragma unroll
-    for (int k = 0; k < M / 2; ++k) {
-      if (k < G) bfly<false>(e[k], o[k], tg[OFF + k], x[k], x[k + M / 2]);
-      else bfly<true>(e[k], o[k], tg[OFF + k - G], x[k], x[k + M / 2]);
-    }
-  }
-};
-template <>
-struct MDit<1> {
-  template <int NT>
-  __device__ __forceinline__ static void run(float2 (&)[1], const float2 (&)[NT]) {}
-};
-
 // Lane constants of stage 2: (tan, cos) of W_(32 m)^(x).
 template <int M>
 __device__ __forceinline__ void hyb_tw(float2 (&tg)[hyb_ntw(M)], const float2 *tw4096, int lane) {

@@ -39,15 +39,25 @@ template <int NP>
 constexpr int wg_team_np(int n) {
   // as many teams as RSK_FS_WG asks for, as far as their LDS regions fit
   const int t = n / elems_fs(n);
-  const int per_team = (RSK_SEQ_POL ? 1 : NP) * (RSK_LDS_PAD > 0 ? n + (n >> RSK_LDS_PAD) : n) +
-                       RSK_TEAM_PAD;
-  const int tw = (RSK_LDS_TW && n > 1) ? n : 1;
+  const int per_team = n + (n >> 4) + 32;
+  const int tw = n > 1 ? n / 2 : 1;
   int teams = RSK_FS_WG / t > 0 ? RSK_FS_WG / t : 1;
   while (teams > 1 && (teams * per_team + tw) * 8 > kLdsBytes) teams /= 2;
   return teams * t;
 }
 constexpr int wg_team(int n) { return wg_team_np<2>(n); }
 constexpr int tile_of(int n) { return wg_team(n) / (n / elems_fs(n)); }
+
+// Pass A's workgroup.  From 2048 points a workgroup of 256 threads is two or
+// one column, whose rows it reads in pieces of 8 or 4 bytes; more columns
+// widen the pieces.  2^23 points (128 MiB): 891 us with 2 columns, 335 with 4,
+// 283 with 8; 2^24 (256 MiB): 3792 with 1, 2130 with 2, 820 with 4.  2^22, whose
+// rows are closer: 213 with 2, 217 with 4, 263 with 8; one pol 331, 113, 139.  (8
+// columns and int16 at 4096 points need registers that 1024 threads leave not.)
+constexpr int wg_a(int n, int nbps) {
+  return n == 2048 ? 512 : (n == 4096 ? (nbps == 16 ? 512 : 1024) : wg_team(n));
+}
+constexpr int tile_a(int n, int nbps) { return wg_a(n, nbps) / (n / elems_fs(n)); }
 
 // Offset within one spectrum's Y of the value (n1, k2 = j + m * T) in the
 // layout [k2 / TBY][n1][k2 % TBY]; linear in m when T is a multiple of TBY.
@@ -62,30 +72,29 @@ __device__ __forceinline__ unsigned y_off(unsigned j, unsigned n1, int m) {
 }
 
 // Pass A for N = N1 * N2 with N1 = R1 * N2 (R1 = 1 or 2).  The four-step
-// twiddle W_N^e, e = n1 * k2 < N, is split as e = h * N1 + r:
-// W_N^(h * N1) = W_N2^h is the sub-transform's own table (already in LDS)
-// and W_N^r, r < N1 <= 4096, is a second LDS table filled from the first
-// N1 entries of the FP64-generated fine table; so each twiddle costs two LDS
-// reads and one complex product (two correctly rounded factors, as with the
-// global two-level table) instead of two scattered global gathers.
+// twiddle of bin k2 = j + m T is W_N^(n1 j) W_N^(n1 m T): a factor of the thread
+// and one common to its column, which TA E of the workgroup's threads compute
+// side by side before the transform into a small LDS table (two of them, used
+// in turn, so that the transform's own barriers order it).  Each factor W_N^e,
+// e = h N1 + r < N, is W_N2^h W_N^r from two FP64-generated tables in global
+// memory.  With those tables in LDS (16 KB) three workgroups shared a CU;
+// without, four do.
 template <int N2, int R1, int NBPS, int NP, bool Y24>
-__global__ __launch_bounds__(wg_team(N2)) void k_fs_a(FsArgs a) {
+__global__ __launch_bounds__(wg_a(N2, NBPS)) void k_fs_a(FsArgs a) {
   static_assert(!Y24 || NP == 2, "24-bit intermediate: two pols");
   constexpr int E = elems_fs(N2);
   constexpr int T = N2 / E;
-  constexpr int TA = tile_of(N2);      // n1 values per workgroup
+  constexpr int TA = tile_a(N2, NBPS);      // n1 values per workgroup
   constexpr int N1C = R1 * N2;
   constexpr int L1 = ilog2(N1C);
-  static_assert(RSK_LDS_TW, "pass A reads the sub-transform table from LDS");
-  static_assert((TA * team_stride<N2, NP>() + TwTab<N2>::LEN + N1C) * 8 <= kLdsBytes,
+  static_assert((TA * fs_stride(N2, TA) + TgTab<N2>::LEN + 2 * TA * E) * 8 <= kLdsBytes,
                 "pass A LDS budget");
   using S = Sample<NBPS, NP>;
   using W = typename S::word;
-  __shared__ float2 lds[TA * team_stride<N2, NP>()];
-  __shared__ float2 twl[TwTab<N2>::LEN];
-  __shared__ float2 twr[N1C];
-  for (int m = threadIdx.x; m < N1C; m += wg_team(N2)) twr[m] = a.twf[m];
-  const float2 *twp = tw_setup<N2, wg_team(N2)>(twl, a.tw);   // also waits for twr
+  __shared__ float2 lds[TA * fs_stride(N2, TA)];
+  __shared__ float2 twt[TgTab<N2>::LEN];
+  __shared__ float2 ctab[2][TA * E];   // [item parity][column of the tile][m]
+  const float2 *twp = tw_setup<N2, wg_a(N2, NBPS)>(twt, a.tw);
 
   const unsigned N1 = N1C;
   const unsigned long long N = (unsigned long long)N1 * N2;
@@ -95,6 +104,7 @@ __global__ __launch_bounds__(wg_team(N2)) void k_fs_a(FsArgs a) {
   const int tid = threadIdx.x;
   int sg = tid % TA;                   // n1 slot: fastest across lanes
   int j = tid / TA;
+  const I8Sign i8s(a.isign);
   constexpr unsigned TBY = tile_of(N1C);  // k2 tile of Y: pass B's workgroup tile
 
   // Item l: (channel cl, buffer b, spectrum sp, tile).  The workgroup takes
@@ -120,6 +130,7 @@ __global__ __launch_bounds__(wg_team(N2)) void k_fs_a(FsArgs a) {
   unsigned l = xcd_remap(blockIdx.x, gridDim.x);
   W raw[E];
   load(l, raw);
+  int par = 0;
   for (;;) {
     // j and sg pass through an empty asm each item, so the compiler
     // recomputes the item's addresses instead of keeping 16 loads' and 16
@@ -128,34 +139,49 @@ __global__ __launch_bounds__(wg_team(N2)) void k_fs_a(FsArgs a) {
     const unsigned ln = l + gridDim.x;   // uniform across the workgroup
     W rawn[E];
     if (ln < items) load(ln, rawn);
+    const unsigned tile = l % tiles;
+    const unsigned n1 = tile * TA + sg;
+    auto wn = [&](unsigned e) {          // W_N^e, e < N
+      return cmul(a.tw[(e >> L1) * (kTwN / N2)], a.twf[e & (N1C - 1)]);
+    };
+    const float2 wj = wn(n1 * (unsigned)j);
+    par ^= 1;
+    static_assert(TA * E <= wg_a(N2, NBPS), "a thread per column factor");
+    if (tid < TA * E) ctab[par][tid] = wn((tile * TA + (unsigned)(tid / E)) * (unsigned)(T * (tid % E)));
     float2 v[NP][E];
+    if constexpr (NBPS == 8) {
+      h2v x[NP][E];
 #pragma unroll
-    for (int m = 0; m < E; ++m) {
-      float2 o[NP];
-      S::cvt(raw[m], o, a.isign);
+      for (int m = 0; m < E; ++m) {
+        x[0][m] = i8_pair_sg<0>((unsigned int)raw[m], i8s);
+        if constexpr (NP == 2) x[NP - 1][m] = i8_pair_sg<1>((unsigned int)raw[m], i8s);
+      }
+      team_fft_h<N2, E, NP, fs_pad(TA)>(x, v, lds + sg * fs_stride(N2, TA), j, twp);
+    } else {
 #pragma unroll
-      for (int p = 0; p < NP; ++p) v[p][m] = o[p];
+      for (int m = 0; m < E; ++m) {
+        float2 o[NP];
+        S::cvt(raw[m], o, a.isign);
+#pragma unroll
+        for (int p = 0; p < NP; ++p) v[p][m] = o[p];
+      }
+      team_fft<N2, E, NP, fs_pad(TA)>(v, lds + sg * fs_stride(N2, TA), j, twp);
     }
-    team_fft<N2, E, NP, TwTab<N2>::TWN>(v, lds + sg * team_stride<N2, NP>(), j, twp);
 
     // Y[cl][(yb0 + b) * Nss + sp][k2 / TBY][n1][k2 % TBY][pol]; offsets
     // within one spectrum (N <= 2^24 values) fit 32 bits
-    const unsigned tile = l % tiles;
     const unsigned cs = l / tiles;
     const unsigned sp = cs % a.Nss;
     const unsigned cb = cs / a.Nss;
     const unsigned b = cb % a.nbat;
     const unsigned cl = cb / a.nbat;
-    const unsigned n1 = tile * TA + sg;
     const unsigned long long spec = (unsigned long long)cl * nsp + (a.yb0 + b) * a.Nss + sp;
     // spectrum `spec` starts at N * NP float2 (24-bit: N * 12 bytes) into Y
     float2 *dst = Y24 ? reinterpret_cast<float2 *>(reinterpret_cast<unsigned int *>(a.work) + spec * N * 3)
                       : a.work + spec * N * NP;
 #pragma unroll
     for (int m = 0; m < E; ++m) {
-      const unsigned k2 = j + m * T;
-      const unsigned e = n1 * k2;          // < N <= 2^24
-      const float2 w = cmul(twl[e >> L1], twr[e & (N1C - 1)]);
+      const float2 w = cmul(ctab[par][sg * E + m], wj);
       const unsigned off = y_off<T, TBY, N1C>(j, n1, m);
       if constexpr (NP == 2) {
         const float2 y0 = cmul(v[0][m], w), y1 = cmul(v[1][m], w);
@@ -186,8 +212,8 @@ void k_fs_b(FsArgs a) {
   constexpr int T = N1 / E;
   constexpr int TB = tile_of(N1);      // k2 values per workgroup
   constexpr int Q = nq<PMODE>();
-  __shared__ float2 lds[TB * team_stride<N1, NP>()];
-  __shared__ float2 twl[TwTab<N1>::LEN];
+  __shared__ float2 lds[TB * fs_stride(N1, TB)];
+  __shared__ float2 twl[TgTab<N1>::LEN];
   const float2 *twp = tw_setup<N1, wg_team(N1)>(twl, a.tw);
 
   const unsigned N2 = a.N2;
@@ -215,7 +241,10 @@ void k_fs_b(FsArgs a) {
   const unsigned sp0 = g * a.na_buf + run * a.sp_run;
   const unsigned sp1 = min(sp0 + a.sp_run, (g + 1) * a.na_buf);
   for (unsigned sp = sp0; sp < sp1; ++sp) {
-    // this workgroup's tile: N1 rows of TB k2 values, contiguous
+    // this workgroup's tile: N1 rows of TB k2 values, contiguous.  (Loading
+    // the next spectrum's values before the last stage of this one changed
+    // nothing: 264 against 254 us per 256 MiB buffer of 2^20 points, 223
+    // against 237 with the 24-bit Y.)
     const unsigned long long e0 = ((unsigned long long)cl * a.Nss * a.ynb + sp) * N +
                                   (unsigned long long)tile * N1 * TB;   // first value of the tile
     const float2 *y = a.work + e0 * NP;
@@ -223,18 +252,18 @@ void k_fs_b(FsArgs a) {
     float2 v[NP][E];
 #pragma unroll
     for (int m = 0; m < E; ++m) {
-      const unsigned long long ev = (unsigned long long)(j + m * T) * TB + sg;
+      const unsigned ev = (unsigned)((j + m * T) * TB + sg);
       if constexpr (NP == 2) {
         float4 t;
         if constexpr (Y24) t = load_y24(y3 + 3 * ev);
-        else t = load_y(reinterpret_cast<const float4 *>(y + ev * NP));
+        else t = load_y(reinterpret_cast<const float4 *>(y) + ev);
         v[0][m] = make_float2(t.x, t.y);
         v[1][m] = make_float2(t.z, t.w);
       } else {
-        v[0][m] = load_y(y + ev * NP);
+        v[0][m] = load_y(y + ev);
       }
     }
-    team_fft<N1, E, NP, TwTab<N1>::TWN>(v, lds + sg * team_stride<N1, NP>(), j, twp);
+    team_fft<N1, E, NP, fs_pad(TB)>(v, lds + sg * fs_stride(N1, TB), j, twp);
 #pragma unroll
     for (int m = 0; m < E; ++m) {
       detect_raw_np<PMODE, NP>(acc[m], v[0][m], v[NP - 1][m]);
@@ -291,12 +320,12 @@ void k_fs_b(FsArgs a) {
   }
 }
 
-int fs_tile_a(int n2) { return (int)(wg_team(n2) / (n2 / elems_fs(n2))); }
+int fs_tile_a(int n2, int nbps) { return tile_a(n2, nbps); }
 int fs_tile_b(int n1) { return (int)(wg_team(n1) / (n1 / elems_fs(n1))); }
 
 template <int N2, int R1, int NBPS>
 static int go_a_r(int np, const FsArgs &a, unsigned nb, hipStream_t s) {
-  constexpr int WGT = wg_team(N2);
+  constexpr int WGT = wg_a(N2, NBPS);
   // 2^18 points: only the 24-bit intermediate comes here (k_fs_a_h.hip)
   if constexpr (N2 == 512 && R1 == 1) {
     if (np != 2 || !a.y24) return 2;
@@ -331,7 +360,7 @@ static int go_a_n(int np, const FsArgs &a, unsigned nb, hipStream_t s) {
 
 int launch_fs_a(int nbps, int np, const FsArgs &a, hipStream_t s) {
   if (a.y24 && np != 2) return 2;
-  const unsigned tiles = a.N1 / fs_tile_a((int)a.N2);
+  const unsigned tiles = a.N1 / fs_tile_a((int)a.N2, nbps);
   const unsigned long long items = (unsigned long long)tiles * a.Nss * a.nbat * a.nch;
   const unsigned long long nb = a.grid_a && a.grid_a < items ? a.grid_a : items;
   // Y's k2 tile: pass B's workgroup tile

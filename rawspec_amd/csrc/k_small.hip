@@ -30,7 +30,7 @@ constexpr int wg_for(int n) {
 template <int N, int NP, int PMODE>
 constexpr int small_lds_f2() {
   constexpr int E = elems_for(N), T = N / E, SLOTS = wg_for(N) / T, Q = nq<PMODE>();
-  constexpr int FFT_F2 = (N > E) ? SLOTS * team_stride<N, NP>() : 1;
+  constexpr int FFT_F2 = (N > E) ? SLOTS * small_stride(N) : 1;
   constexpr int RED_F2 = SLOTS >= 2 ? ((SLOTS / 2) * Q * N + 1) / 2 : 1;
   return FFT_F2 > RED_F2 ? FFT_F2 : RED_F2;
 }
@@ -56,7 +56,7 @@ void k_small(SmallArgs a) {
   using S = Sample<NBPS, NP>;
   using W = typename S::word;
   __shared__ float2 lds[LDS_F2];
-  __shared__ float2 twl[TwTab<N>::LEN];
+  __shared__ float2 twl[TgTab<N>::LEN];
 
   // Workgroup -> (channel, first group, chunk).  gpw groups per workgroup
   // (each with spg = SLOTS/gpw slots) when groups are short; otherwise one
@@ -76,6 +76,7 @@ void k_small(SmallArgs a) {
   const bool gvalid = g < a.Ng;
 
   const float2 *twp = tw_setup<N, WG>(twl, a.tw);
+  const I8Sign i8s(a.isign);
   const W *src = reinterpret_cast<const W *>(a.in + (unsigned long long)c * a.chan_stride);
   // transform length (samples per spectrum, bins per output spectrum)
   const unsigned NT = BS ? a.nt : (unsigned)N;
@@ -111,14 +112,28 @@ void k_small(SmallArgs a) {
 #pragma unroll
       for (int m = 0; m < E; ++m) raw[m] = src[sbase + j + m * T];
     }
-    // one thread per int8 transform: samples offset by 128, removed from bin
-    // 0 (the thread's element 0) after the single-stage transform
-    constexpr bool kOffset = T == 1 && NBPS == 8 && !BS;
+    // int8 samples become FP16 pairs; several threads per transform: up to the
+    // first exchange; one thread: dft_pairs
+    constexpr bool kPairs = NBPS == 8 && !BS;
+    if constexpr (kPairs) {
+      h2v x[NP][E];
+#pragma unroll
+      for (int m = 0; m < E; ++m) {
+        x[0][m] = i8_pair_sg<0>((unsigned int)raw[m], i8s);
+        if constexpr (NP == 2) x[NP - 1][m] = i8_pair_sg<1>((unsigned int)raw[m], i8s);
+      }
+      if constexpr (T > 1) {
+        team_fft_h<N, E, NP, kSmallPad, (T <= 64)>(x, v, lds + slot * small_stride(N), j, twp);
+      } else {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) dft_pairs<N>(x[p], v[p]);
+      }
+    }
 #pragma unroll
     for (int m = 0; m < E; ++m) {
+      if constexpr (kPairs) break;
       float2 o[NP];
-      if constexpr (kOffset) S::cvt_offset(raw[m], o, a.isign);
-      else S::cvt(raw[m], o, a.isign);
+      S::cvt(raw[m], o, a.isign);
 #pragma unroll
       for (int p = 0; p < NP; ++p) v[p][m] = o[p];
     }
@@ -137,7 +152,8 @@ void k_small(SmallArgs a) {
       }
     }
     // a team is T consecutive threads: within one wavefront when T <= 64
-    team_fft<N, E, NP, TwTab<N>::TWN, (T <= 64)>(v, lds + slot * team_stride<N, NP>(), j, twp);
+    if constexpr (!kPairs)
+      team_fft<N, E, NP, kSmallPad, (T <= 64)>(v, lds + slot * small_stride(N), j, twp);
     if constexpr (BS) {
 #pragma unroll
       for (int m = 0; m < E; ++m) {
@@ -153,20 +169,13 @@ void k_small(SmallArgs a) {
       // keep those values live in between)
       unsigned zw;
       asm volatile("v_mov_b32 %0, 0" : "=v"(zw));
-      team_fft<N, E, NP, TwTab<N>::TWN, (T <= 64)>(v, lds + slot * team_stride<N, NP>(), j, twp + zw);
+      team_fft<N, E, NP, kSmallPad, (T <= 64)>(v, lds + slot * small_stride(N), j, twp + zw);
 #pragma unroll
       for (int m = 0; m < E; ++m) {
         const unsigned k = (unsigned)(j + m * T);
         const float2 ck = k < NT ? a.chirp[k + zt] : make_float2(0.0f, 0.0f);
 #pragma unroll
         for (int p = 0; p < NP; ++p) v[p][m] = cmul(make_float2(v[p][m].x, -v[p][m].y), ck);
-      }
-    }
-    if constexpr (kOffset) {
-#pragma unroll
-      for (int p = 0; p < NP; ++p) {
-        v[p][0].x -= 128.0f * N;
-        v[p][0].y -= a.isign * (128.0f * N);
       }
     }
     if (valid) {

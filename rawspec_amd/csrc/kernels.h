@@ -20,7 +20,9 @@ constexpr int kHybOperands = 2 * 4 * 2 * 64 * 16 / 8;
 constexpr int dit_off(int m) { return m <= 2 ? 0 : dit_off(m / 2) + (m / 2 <= 4 ? 1 : m / 8); }
 constexpr int hyb_ntw(int M) { return M == 32 ? 9 : (M <= 2 ? 1 : dit_off(M) + (M >= 8 ? M / 4 : 1)); }
 constexpr int hyb_tw_off(int M) { return M <= 2 ? 0 : hyb_tw_off(M / 2) + 64 * hyb_ntw(M / 2); }
-constexpr int kTwTotal = kTwN + kHybOperands + hyb_tw_off(64);   // float2 of the device table
+// Then the (tan, cos) of W_4096^m, m < 2048 (fft_device.h's stages).
+constexpr int kTgOff = kTwN + kHybOperands + hyb_tw_off(64);
+constexpr int kTwTotal = kTgOff + kTwN / 2;   // float2 of the device table
 
 // Fused small-N path (N <= 4096): unpack -> FFT -> detect -> integrate a
 // chunk of `chunk` spectra.  Workgroup b covers channel b / bpc and either
@@ -123,7 +125,7 @@ struct IcsArgs {
 // Query functions used by the host-side planner.
 int small_wg(int n);            // threads per workgroup of the small kernel
 int small_slots(int n);         // spectra processed concurrently per workgroup
-int fs_tile_a(int n2);          // n1 values per pass-A workgroup
+int fs_tile_a(int n2, int nbps);  // n1 values per workgroup of the vector pass A
 int fs_tile_b(int n1);          // k2 values per pass-B workgroup
 
 // Launchers; return 0 on success, non-zero for an unsupported shape or a

@@ -30,7 +30,7 @@
 // scaling on the detected power.
 #pragma once
 
-#include <hip/hip_runtime.h>
+#include "fft_device.h"
 
 namespace rsk {
 
@@ -152,7 +152,6 @@ __device__ __forceinline__ void dft1024(const float2 (&x)[4][4], const Dft1024K 
 // of roughly 6e-3 / sqrt(K) over a floor near 1.5e-4 (measured on a numpy
 // emulation of these roundings with int8 noise and a strong tone).  Inputs are
 // used unscaled: |stage-1 result| <= 32 * 127 * sqrt(2) < 2^13.
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 
 // Constants of the unsplit transform: B operands of the 32-point DFT matrix
 // (real-output and imaginary-output halves, 4 K-blocks) and the twiddles

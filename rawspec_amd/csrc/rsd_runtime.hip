@@ -244,6 +244,10 @@ void hybrid_tables(std::vector<float2> &t) {
     for (int k = 0; k < 2; ++k) put(32, 3 + k, lane, 16, c + 32 * (h + 2 * k));
     for (int k = 0; k < 4; ++k) put(32, 5 + k, lane, 32, c + 32 * (h + 2 * k));
   }
+  for (int m = 0; m < rsk::kTwN / 2; ++m) {
+    const double ang = -2.0 * M_PI * (double)m / (double)rsk::kTwN;
+    t[rsk::kTgOff + m] = make_float2((float)(sin(ang) / cos(ang)), (float)cos(ang));
+  }
 }
 
 }  // namespace
