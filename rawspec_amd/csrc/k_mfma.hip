@@ -267,33 +267,6 @@ __global__ __launch_bounds__(64 * kMfmaWaves, (NBPS == 16 && PMODE != 1) ? 1 : 2
 }
 
 // ---- an 8-point product fused into the unsplit 1024-point kernel ----------
-// Forward 8-point DFT in place, natural order: radix 2, decimation in
-// frequency, W8 = exp(-2 pi i / 8).
-__device__ __forceinline__ void dft8(float2 (&x)[8]) {
-  constexpr float r = 0.70710678118654752f;
-  const float2 a0 = cadd(x[0], x[4]), a1 = cadd(x[1], x[5]);
-  const float2 a2 = cadd(x[2], x[6]), a3 = cadd(x[3], x[7]);
-  const float2 b0 = csub(x[0], x[4]), d1 = csub(x[1], x[5]);
-  const float2 d2 = csub(x[2], x[6]), d3 = csub(x[3], x[7]);
-  // times W8^1 = (1 - i) r, W8^2 = -i, W8^3 = (-1 - i) r
-  const float2 b1 = make_float2((d1.x + d1.y) * r, (d1.y - d1.x) * r);
-  const float2 b2 = make_float2(d2.y, -d2.x);
-  const float2 b3 = make_float2((d3.y - d3.x) * r, -(d3.x + d3.y) * r);
-  // the two 4-point halves: even outputs from a, odd outputs from b
-  const float2 c0 = cadd(a0, a2), c1 = cadd(a1, a3), c2 = csub(a0, a2), e3 = csub(a1, a3);
-  const float2 c3 = make_float2(e3.y, -e3.x);
-  const float2 g0 = cadd(b0, b2), g1 = cadd(b1, b3), g2 = csub(b0, b2), f3 = csub(b1, b3);
-  const float2 g3 = make_float2(f3.y, -f3.x);
-  x[0] = cadd(c0, c1);
-  x[4] = csub(c0, c1);
-  x[2] = cadd(c2, c3);
-  x[6] = csub(c2, c3);
-  x[1] = cadd(g0, g1);
-  x[5] = csub(g0, g1);
-  x[3] = cadd(g2, g3);
-  x[7] = csub(g2, g3);
-}
-
 template <int CTRL, int BANKS>
 __device__ __forceinline__ float dpp_f(float old, float src) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old),
@@ -519,20 +492,20 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void k_small_mfma_u(SmallArgs a
         uint4 w[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) w[k] = p4[k];
-        float2 x0[8], x1[8];
+        h2v x0[8], x1[8];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          const h2v s00 = __builtin_bit_cast(h2v, w[k].x), s01 = __builtin_bit_cast(h2v, w[k].y);
-          const h2v s10 = __builtin_bit_cast(h2v, w[k].z), s11 = __builtin_bit_cast(h2v, w[k].w);
-          x0[2 * k] = make_float2((float)s00[0], (float)s00[1]);
-          x1[2 * k] = make_float2((float)s01[0], (float)s01[1]);
-          x0[2 * k + 1] = make_float2((float)s10[0], (float)s10[1]);
-          x1[2 * k + 1] = make_float2((float)s11[0], (float)s11[1]);
+          x0[2 * k] = __builtin_bit_cast(h2v, w[k].x);
+          x1[2 * k] = __builtin_bit_cast(h2v, w[k].y);
+          x0[2 * k + 1] = __builtin_bit_cast(h2v, w[k].z);
+          x1[2 * k + 1] = __builtin_bit_cast(h2v, w[k].w);
         }
-        dft8(x0);
-        dft8(x1);
+        const Bins8 b0 = dft8_h(x0), b1 = dft8_h(x1);
 #pragma unroll
-        for (int b = 0; b < 8; ++b) detect_raw<PMODE>(a8[b], x0[b].x, x0[b].y, x1[b].x, x1[b].y);
+        for (int b = 0; b < 8; ++b) {
+          const float2 y0 = b0.bin(b), y1 = b1.bin(b);
+          detect_raw<PMODE>(a8[b], y0.x, y0.y, y1.x, y1.y);
+        }
         __builtin_amdgcn_sched_barrier(0);             // one spectrum's samples live at a time
       }
       constexpr int V = 8 * Q;
@@ -569,6 +542,23 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void k_small_mfma_u(SmallArgs a
     for (int q = 0; q < Q; ++q) sw[q * kSmRow + jo + (jo >> 5)] = acc[r][q];
   }
   __syncthreads();
+  if (!a.direct && a.G % kMfmaWaves == 0) {
+    // the workgroup's chunks belong to one group: one partial sum for all,
+    // added in chunk order (a quarter of the partial sums' traffic; the
+    // launch that adds them 15.6 -> 6 us on 64 channels of Stokes)
+    const unsigned gp = a.G / kMfmaWaves;
+    float *dst = a.part + ((((unsigned long long)c * a.Ng + g) * gp + chunk / kMfmaWaves) * Q) * N;
+    if (!valid) return;                            // whole workgroups only
+    for (int idx = threadIdx.x; idx < Q * N; idx += 64 * kMfmaWaves) {
+      const int q = idx >> 10, jo = idx & (N - 1);
+      const float *p = st + q * kSmRow + jo + (jo >> 5);
+      float v = p[0];
+#pragma unroll
+      for (int w = 1; w < kMfmaWaves; ++w) v += p[w * (Q * kSmRow)];
+      dst[idx] = v;
+    }
+    return;
+  }
   if (!valid) return;
   for (int q = 0; q < Q; ++q) {
     float *dst;

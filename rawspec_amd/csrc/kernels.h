@@ -156,7 +156,8 @@ int launch_small_mfma(int n, int nbps, int np, int pmode, const SmallArgs &a, un
                       hipStream_t s);
 // The same with unsplit FP16 operands (int8 samples only): a third of the
 // matrix instructions, error of order 6e-3 / sqrt(spectra integrated) over a
-// floor near 1.5e-4, for products that integrate enough spectra.
+// floor near 1.5e-4, for products that integrate enough spectra.  With G a
+// multiple of 4 and not direct it leaves G / 4 partial sums per group.
 int launch_small_mfma_u(int n, int nbps, int np, int pmode, const SmallArgs &a, unsigned items,
                         hipStream_t s);
 // Matrix-core pass A (N1 = N2 = 1024, int8, two pols): k_fs_a's contract;

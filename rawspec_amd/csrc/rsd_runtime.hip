@@ -1008,7 +1008,8 @@ static int run_small(rsd_ctx *d, int i, const uint8_t *in, float isign, float ga
     r.acc = pp.d_acc;
     r.Nc = c.Nc;
     r.Ng = pp.Ng;
-    r.G = a.G;
+    // the unsplit matrix-core kernel adds its workgroup's four chunks
+    r.G = mf && d->mfma == 1 && pp.m_unsplit && a.G % 4 == 0 ? a.G / 4 : a.G;
     r.Q = (unsigned)pp.Q;
     r.N = pp.p.Nt;
     r.scale = scale;
