@@ -417,49 +417,45 @@ int launch_fs_b(int np, int pmode, const FsArgs &a, hipStream_t s) {
   return 2;
 }
 
-// One thread per value of the launch's sums: the ns partial sums in run
+// One thread per four values of the launch's sums: the ns partial sums in run
 // order, then the finish k_fs_b applies to its own sums (same scale, same
-// internal-accumulator block, same shifted output position).
-__global__ __launch_bounds__(256) void k_fs_b_reduce(FsArgs a, unsigned Q, unsigned TB) {
-  const unsigned N1 = a.N1, N2 = a.N2, tiles = N2 / TB;
+// internal-accumulator block, same shifted output position).  Bound by the
+// partial sums' bytes: 16-byte loads, four runs in flight, and shifts for the
+// power-of-two sizes (single floats placed by 64-bit divisions took 28 us for
+// four runs of 2^18 points x 3 x 4 sums, 50 MB).
+template <int Q>
+__global__ __launch_bounds__(256) void k_fs_b_reduce(FsArgs a, unsigned lTB) {
+  using f4 = float __attribute__((ext_vector_type(4)));
+  const unsigned N1 = a.N1, N2 = a.N2, lN1 = 31 - __builtin_clz(N1), TB = 1u << lTB;
   const unsigned long long N = (unsigned long long)N1 * N2;
-  const unsigned long long total = (unsigned long long)a.Ng * a.nch * tiles * Q * N1 * TB;
-  for (unsigned long long idx = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-       idx < total; idx += (unsigned long long)gridDim.x * blockDim.x) {
-    // idx runs over [Ng][nch][tiles][Q][N1][TB], one run's block of partb
-    const unsigned sg = (unsigned)(idx % TB);
-    unsigned long long r = idx / TB;
-    const unsigned k1 = (unsigned)(r % N1);
-    r /= N1;
-    const unsigned q = (unsigned)(r % Q);
-    r /= Q;
-    const unsigned tile = (unsigned)(r % tiles);
-    r /= tiles;
-    const unsigned cl = (unsigned)(r % a.nch);
-    const unsigned g = (unsigned)(r / a.nch);
-    // runs in order, eight loads in flight (a chain of 64 single loads took
-    // 30 us, as long as pass B)
-    float sum = 0.0f;
-    unsigned run = 0;
-    for (; run + 8 <= a.ns; run += 8) {
-      float v[8];
+  // idx runs over [tiles][Q][N1][TB], one (group, channel)'s block of a run
+  const unsigned idx = (blockIdx.x * 256 + threadIdx.x) * 4;
+  const unsigned sg = idx & (TB - 1), k1 = (idx >> lTB) & (N1 - 1);
+  const unsigned tq = idx >> (lTB + lN1), q = tq % Q, tile = tq / Q;
+  const unsigned rows = a.Ng * a.nch;
+  const unsigned long long total = (unsigned long long)rows * Q * N;
+  for (unsigned gc = blockIdx.y; gc < rows; gc += gridDim.y) {
+    const unsigned g = gc / a.nch, c = a.c0 + (gc - g * a.nch);
+    const float *p = a.partb + (unsigned long long)gc * Q * N + idx;
+    f4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (unsigned run = 0; run < a.ns; run += 4) {
+      f4 v[4];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = load_acc(a.partb + (run + u) * total + idx);
+      for (unsigned u = 0; u < 4; ++u)
+        if (run + u < a.ns) v[u] = *reinterpret_cast<const f4 *>(p + (run + u) * total);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) sum += v[u];
+      for (unsigned u = 0; u < 4; ++u)
+        if (run + u < a.ns) sum += v[u];
     }
-    for (; run < a.ns; ++run) sum += load_acc(a.partb + run * total + idx);
-    float v = sum * a.scale;
-    const unsigned c = a.c0 + cl;
-    float *ie = a.acc_int + ((((unsigned long long)g * a.Nc + c) * tiles + tile) * Q + q) * N1 * TB +
-                (unsigned long long)k1 * TB + sg;
-    if (a.mode == FS_MID || a.mode == FS_LAST) v += load_acc(ie);
+    f4 v = sum * a.scale;
+    f4 *ie = reinterpret_cast<f4 *>(a.acc_int + (((unsigned long long)g * a.Nc + c) * Q * N + idx));
+    if (a.mode == FS_MID || a.mode == FS_LAST) v += *ie;
     if (a.mode == FS_FIRST || a.mode == FS_MID) {
-      store_acc(ie, v);
+      *ie = v;
     } else {
-      const unsigned k2 = tile * TB + sg;
-      a.acc[((unsigned long long)g * Q * a.Nc + c) * N + k2 + (unsigned long long)q * a.Nc * N +
-            (unsigned long long)N2 * ((k1 + N1 / 2) & (N1 - 1))] = v;
+      float *o = a.acc + (((unsigned long long)g * Q + q) * a.Nc + c) * N + tile * TB + sg +
+                 (unsigned long long)N2 * ((k1 + N1 / 2) & (N1 - 1));
+      *reinterpret_cast<f4 *>(o) = v;
     }
   }
 }
@@ -468,11 +464,13 @@ int launch_fs_b_reduce(int pmode, const FsArgs &a, hipStream_t s) {
   if (a.ns < 2 || !runs_ok(a)) return 2;
   const unsigned Q = pmode == 1 ? 1u : 4u;
   const unsigned TB = (unsigned)fs_tile_b((int)a.N1);
-  const unsigned long long total = (unsigned long long)a.Ng * a.nch * (a.N2 / TB) * Q * a.N1 * TB;
-  if (total == 0) return 2;
-  unsigned long long nb = (total + 255) / 256;
-  if (nb > 16384) nb = 16384;
-  hipLaunchKernelGGL(k_fs_b_reduce, dim3((unsigned)nb), dim3(256), 0, s, a, Q, TB);
+  const unsigned long long rows = (unsigned long long)a.Ng * a.nch;
+  const unsigned nb = a.N1 * a.N2 / 1024 * Q;    // N1, N2 >= 64
+  if (rows == 0 || rows > 0xffffffffull || nb == 0) return 2;
+  const dim3 grid(nb, rows < 65535 ? (unsigned)rows : 65535u);
+  const unsigned lTB = (unsigned)__builtin_ctz(TB);
+  if (Q == 1) hipLaunchKernelGGL((k_fs_b_reduce<1>), grid, dim3(256), 0, s, a, lTB);
+  else hipLaunchKernelGGL((k_fs_b_reduce<4>), grid, dim3(256), 0, s, a, lTB);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 

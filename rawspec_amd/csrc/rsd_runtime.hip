@@ -124,13 +124,14 @@ constexpr size_t kLaneMinBytes = (size_t)64 << 20;
 #define RSD_HOLD_MB 8192
 #endif
 constexpr size_t kHoldBytes = (size_t)RSD_HOLD_MB << 20;
-// Vector pass B: workgroups per CU a launch aims for, splitting each dump
-// group's spectra into runs when its (k2 tile, group, channel) workgroups
-// are fewer; the fewest spectra a run integrates; the CU count the planner
-// sizes the runs' partial sums for (launches use the device's own count,
-// capped by what was allocated).
+// Vector pass B (fsb_runs): workgroups per CU a split launch aims for; the
+// workgroups per 2 CUs from which a launch stays whole; the partial sums
+// whose traffic costs as much as a spectrum of a run; the CU count the
+// planner sizes the runs' partial sums for (launches use the device's own
+// count, capped by what was allocated).
 constexpr unsigned kFsbWgPerCu = 4;
-constexpr unsigned kFsbMinRun = 1;
+constexpr unsigned kFsbFull = 3;
+constexpr unsigned long long kFsbRunSums = 1ull << 20;
 constexpr unsigned kPlanCus = 256;
 
 bool is_pow2(unsigned n) { return n && !(n & (n - 1)); }
@@ -591,26 +592,32 @@ static unsigned fs_chunk_for(const rsd_ctx *d, const ProdPlan &pp, unsigned kb) 
 }
 
 // Runs each dump group of a vector pass-B launch with na_buf spectra per
-// group is split into, for cus compute units: enough for about kFsbWgPerCu
-// workgroups per CU where the (k2 tile, group, channel) workgroups of all
-// Nc channels are fewer, each run at least kFsbMinRun spectra.  A workgroup
-// otherwise integrates its whole group in turn: a 2^13-point product over 8
-// channels is 128 workgroups, each summing thousands of spectra.  The count
-// depends on the context's channels, not on a launch's channel chunk, so
-// every path over the same buffers (batched, held, allocation-free with
-// its smaller chunks) adds the same runs in the same order.
+// group is split into, for cus compute units.  A workgroup otherwise
+// integrates its whole group in turn: a 2^13-point product over 8 channels is
+// 32 workgroups, each summing thousands of spectra.  A split pays while the
+// (k2 tile, group, channel) workgroups of all Nc channels are fewer than
+// kFsbFull per 2 CUs: at 1.5 per CU and more it gained nothing (2^17 points,
+// 32 spectra, 12 channels 0.9..1.05x), at one 1.1..1.24x.  Runs cost a launch and
+// their partial sums' traffic, which grows with their number, as their gain
+// shrinks: the time n t / ns + ns c is least at ns^2 = n t / c, about n
+// kFsbRunSums / (sums of the launch); twice and four times that lost up to
+// 12% on 4 sums a point.  The launch (5 us) is worth 3 spectra of 128 points saved,
+// 2 of 256.  (2^16 points, 2 channels, 4 spectra: 24.5 -> 16.3 us; 2^14, 2
+// channels, 32 spectra of 4 sums: 87 -> 23; 2^18, 1 channel of 4 spectra in 3
+// groups of 4 sums stays whole: 33 us, split 53.)  The count depends on the
+// context's channels, not on a launch's channel chunk, so every path over the
+// same buffers (batched, held, allocation-free with its smaller chunks) adds
+// the same runs in the same order.
 static unsigned fsb_runs(const ProdPlan &pp, unsigned cus, unsigned Nc, unsigned na_buf) {
   const unsigned long long base =
       (unsigned long long)(pp.N2 / (unsigned)rsk::fs_tile_b((int)pp.N1)) * pp.Ng * Nc;
-  const unsigned long long target = (unsigned long long)cus * kFsbWgPerCu;
-  if (base == 0 || base >= target) return 1;
-  unsigned long long ns = (target + base - 1) / base;
-  // groups of two or three spectra save less than the runs' launch costs; from
-  // four on a spectrum per run is best (2^16 points, 2 channels, 4 spectra: 52
-  // us whole, 38 in runs of two, 28 in runs of one)
-  const unsigned maxr = na_buf < 4 ? 1 : na_buf / kFsbMinRun;
-  if (ns > maxr) ns = maxr;
-  return ns < 1 ? 1u : (unsigned)ns;
+  if (base == 0 || 2 * base >= (unsigned long long)cus * kFsbFull) return 1;
+  unsigned long long ns = ((unsigned long long)cus * kFsbWgPerCu + base - 1) / base;
+  if (ns > na_buf) ns = na_buf;
+  const unsigned long long sums = (unsigned long long)pp.Q * pp.p.Nt * pp.Ng * Nc;
+  while (ns > 1 && ns * ns * sums > na_buf * kFsbRunSums) --ns;
+  if (ns < 2 || (na_buf - (na_buf + ns - 1) / ns) * pp.N1 < 3 * 128) return 1;
+  return (unsigned)ns;
 }
 
 // floats of partial sums a pass-B launch split into ns runs writes
