@@ -29,7 +29,7 @@ ARCH = os.environ.get("RAWSPEC_AMD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CC = os.environ.get("CC", "gcc")
 
-HIP_SOURCES = ["rsd_runtime.hip", "k_small.hip", "k_small_h.hip", "k_fourstep.hip", "k_fs_a_h.hip", "k_mfma.hip", "k_misc.hip"]
+HIP_SOURCES = ["rsd_runtime.hip", "k_small.hip", "k_small_h.hip", "k_small_r.hip", "k_fourstep.hip", "k_fs_a_h.hip", "k_mfma.hip", "k_misc.hip"]
 C_SOURCES = ["rawspec_api.c", "raw_header.c", "fb_header.c"]
 
 HIP_FLAGS = [

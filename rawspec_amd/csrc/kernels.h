@@ -48,7 +48,8 @@ struct SmallArgs {
   float *part;                    // [Nc][Ng][G][Q][N] unscaled, FFT-shifted
   const float2 *tw;               // W_4096^m, m < 4096, and behind it kTwTotal's rest
   // transform length: the kernel's N, or for a product whose length is not
-  // a power of two (Bluestein, N >= 2 nt - 1) nt with its tables
+  // a power of two (Bluestein, N >= 2 nt - 1) nt with its tables; k_small_r has
+  // its twiddles W_nt^n in chirp
   unsigned nt;
   const float2 *chirp;            // c[n] = exp(-i pi n^2 / nt), n < nt
   const float2 *bsk;              // FFT_N of the wrapped conjugate chirp, over N
@@ -107,6 +108,14 @@ struct FsArgs {
   float *partb;
 };
 
+// Mixed-radix small kernel (k_small_r.hip): elements per thread, stages with
+// their radices and division constants, spectra and threads per workgroup.
+constexpr unsigned kRMaxStages = 5, kRMinN = 40;
+struct RPlan {
+  unsigned e, n, slots, threads;
+  unsigned r[kRMaxStages], magic[kRMaxStages];
+};
+
 struct ReduceArgs {
   const float *part;
   float *acc;
@@ -149,6 +158,11 @@ int launch_fs_b_reduce(int pmode, const FsArgs &a, hipStream_t s);
 int small_h_ok(int n, unsigned na_buf);
 int launch_small_h(int n, int nbps, int np, int pmode, const SmallArgs &a, unsigned nblocks, int solo,
                    int waves, hipStream_t s);
+// Lengths 2^a 3^b and 2^a 5^b (k_small_r.hip): r_plan fills rp, or returns false
+// where the length is Bluestein's; a.chirp holds W_N^n.
+bool r_plan(unsigned n, int np, RPlan &rp);
+int launch_small_r(int nbps, int np, int pmode, const SmallArgs &a, const RPlan &rp, unsigned nblocks,
+                   hipStream_t s);
 // Matrix-core fused small kernel (N = 1024, two pols): one wavefront per
 // (channel, group, chunk) item, items = Nc * Ng * G, gpw must be 1.
 int small_mfma_ok(int n, int np);

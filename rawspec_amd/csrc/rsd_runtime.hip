@@ -60,6 +60,10 @@ struct ProdPlan {
   unsigned bs_m;
   float2 *d_chirp;
   float2 *d_bsk;
+  // such a length of the form 2^a 3^b or 2^a 5^b: the mixed-radix kernel, with
+  // d_chirp its twiddles W_N^n (d_bsk and bs_m not used)
+  int r_ok;
+  rsk::RPlan rp;
   // small path
   unsigned na_buf, Ng, chunk, G, gpw, spg, bpc;
   int direct;
@@ -350,12 +354,13 @@ struct ProfScope {
 };
 
 static void plan_small(rsd_ctx *d, ProdPlan &pp) {
-  const unsigned slots = (unsigned)rsk::small_slots((int)(pp.bs ? pp.bs_m : pp.p.Nt));
+  const unsigned n = pp.bs ? pp.bs_m : pp.p.Nt;
+  const unsigned vslots = (unsigned)rsk::small_slots((int)n), slots = pp.r_ok ? pp.rp.slots : vslots;
+  const unsigned wg = pp.r_ok ? pp.rp.threads : (unsigned)rsk::small_wg((int)n);
   const unsigned Nc = d->cfg.Nc;
   pp.na_buf = pp.p.Na < pp.p.Nss ? pp.p.Na : pp.p.Nss;
   pp.Ng = pp.p.Nss / pp.na_buf;
   pp.chunk = pp.na_buf;
-  const unsigned n = pp.bs ? pp.bs_m : pp.p.Nt;
   // Split long groups over workgroups until the launch fills the device
   // (by default about 2048 workgroups for 256 CUs), keeping >= one spectrum
   // per slot.  From 2048 points a workgroup's one or two slots hold a CU's
@@ -364,7 +369,7 @@ static void plan_small(rsd_ctx *d, ProdPlan &pp) {
   // against 141 us).
   const unsigned long long target = n >= 2048 ? pp.t_target / 4 : pp.t_target;
   while ((unsigned long long)Nc * pp.Ng * (pp.na_buf / pp.chunk) < target && pp.chunk % 2 == 0 &&
-         pp.chunk / 2 >= slots)
+         pp.chunk / 2 >= (slots > vslots ? slots : vslots))
     pp.chunk /= 2;
   pp.G = pp.na_buf / pp.chunk;
   pp.direct = pp.G == 1;
@@ -382,7 +387,7 @@ static void plan_small(rsd_ctx *d, ProdPlan &pp) {
     // more slots for a long group where that makes too few wavefronts (8
     // points in dumps of 1024 spectra, 64 MiB: 17 against 47 us; shorter
     // dumps fill the device as they are and lose by it, 16 against 22)
-    const unsigned long long fill = 8192ull * 64 / (unsigned)rsk::small_wg((int)n);
+    const unsigned long long fill = 8192ull * 64 / wg;
     while (spg < slots && pp.chunk >= 8 * spg &&
            (unsigned long long)Nc * ((pp.Ng + slots / spg - 1) / (slots / spg)) < fill)
       spg <<= 1;
@@ -699,6 +704,20 @@ static bool f8_pair(const rsd_ctx *d, const ProdPlan &a, const ProdPlan &b) {
 }
 static bool f8_on(const rsd_ctx *d) { return d->f8_a >= 0 && d->mfma == 1; }
 
+// Whether a length of the mixed-radix kernel's form is better there than in
+// Bluestein's: nearly always, but a buffer of few points waits for the chain of
+// one transform, which more threads with less work each make shorter (4
+// channels, 1152 points, dumps of 8 spectra of 4 sums: 1 MiB 29 against 18 us,
+// 4 MiB 34 against 61, 32 MiB 95 against 298; one sum 18 against 16, 21 against
+// 35, 74 against 187; 2000 points, one sum: 14 against 16, 17 against 22, 68
+// against 157).  The lines are 2^18 points of one polarisation, 2^19 of two,
+// 2^20 of two with four sums.  Four sums of the shortest lengths leave too many
+// sums to write (48 points 267 against 216 us, 80 points 120 against 485).
+static bool r_pays(const rsd_config *cfg, const ProdPlan &pp) {
+  const unsigned long long points = (unsigned long long)cfg->Nc * pp.p.Nss * pp.p.Nt;
+  return points >= (1ull << 17) * cfg->Np * (pp.Q == 1 ? 2 : 4) && pp.p.Nt >= (pp.Q == 1 ? 40u : 80u);
+}
+
 static int plan_all(const rsd_config *cfg, rsd_ctx *d) {
   d->dev = cfg->gpu_index;
   d->cfg = *cfg;
@@ -728,9 +747,11 @@ static int plan_all(const rsd_config *cfg, rsd_ctx *d) {
     pp.Q = pp.p.npolout == 1 ? 1 : 4;
     pp.bs = !is_pow2(N);
     pp.bs_m = N;
+    pp.r_ok = 0;
     if (pp.bs) {
       pp.bs_m = 1;
       while (pp.bs_m < 2 * N - 1) pp.bs_m <<= 1;
+      pp.r_ok = r_pays(cfg, pp) && rsk::r_plan(N, (int)cfg->Np, pp.rp);
     }
     pp.small = pp.bs || N <= (unsigned)rsk::kTwN;
     pp.t_target = 2048;
@@ -768,7 +789,7 @@ static size_t plan_bytes(const rsd_ctx *d) {
   for (unsigned i = 0; i < d->cfg.No; ++i) {
     const ProdPlan &pp = d->pp[i];
     b += pp.acc_len * sizeof(float) + pp.ics_len * sizeof(float);
-    if (pp.bs) b += ((size_t)pp.p.Nt + pp.bs_m) * sizeof(float2);
+    if (pp.bs) b += ((size_t)pp.p.Nt + (pp.r_ok ? 0 : pp.bs_m)) * sizeof(float2);
     if (!pp.small) {
       b += (size_t)pp.N1 * sizeof(float2);
       if (pp.p.Nis > 1) b += pp.acc_len * sizeof(float);
@@ -820,7 +841,11 @@ static int create_impl(const rsd_config *cfg, rsd_ctx *d) {
       RSD_CHECK(hipMemcpy(pp.d_twf, f.data(), f.size() * sizeof(float2), hipMemcpyHostToDevice));
       if (pp.p.Nis > 1 && alloc_zero((void **)&pp.d_acc_int, pp.acc_len * sizeof(float))) return 1;
     }
-    if (pp.bs) {
+    if (pp.r_ok) {
+      std::vector<float2> t = twiddles(N, N, 1);
+      RSD_CHECK(hipMalloc(&pp.d_chirp, t.size() * sizeof(float2)));
+      RSD_CHECK(hipMemcpy(pp.d_chirp, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice));
+    } else if (pp.bs) {
       std::vector<float2> ch, bk;
       bluestein_tables(N, pp.bs_m, ch, bk);
       RSD_CHECK(hipMalloc(&pp.d_chirp, ch.size() * sizeof(float2)));
@@ -1005,7 +1030,9 @@ static int run_small(rsd_ctx *d, int i, const uint8_t *in, float isign, float ga
     const unsigned long long nb = (unsigned long long)pp.bpc * c.Nc;
     if (nb > 0x7fffffffull) return 1;
     ProfScope ps(d, i, "k_small", pp.p.Nt, s);
-    if (rsk::launch_small((int)pp.bs_m, (int)c.Nbps, (int)c.Np, pp.p.npolout, a, (unsigned)nb,
+    if (pp.r_ok) {
+      if (rsk::launch_small_r((int)c.Nbps, (int)c.Np, pp.p.npolout, a, pp.rp, (unsigned)nb, s)) return 1;
+    } else if (rsk::launch_small((int)pp.bs_m, (int)c.Nbps, (int)c.Np, pp.p.npolout, a, (unsigned)nb,
                           s))
       return 1;
   }
