@@ -12,7 +12,9 @@ fallback implementation.
 """
 from __future__ import annotations
 
+import atexit
 import ctypes as C
+import itertools
 import os
 
 import numpy as np
@@ -227,16 +229,30 @@ def lib():
     return _lib
 
 
-class DevicePointer(int):
-    """A device address (an int) that keeps the context owning the memory
-    alive: an array made from it (through __cuda_array_interface__, which the
-    consumer holds on to) must not outlive the buffers, which are freed when
-    the Spectrometer is collected."""
+# Contexts that were collected (not closed) after handing out device addresses:
+# an array made from such an address does not hold the context, and the cyclic
+# collector, which frees a dropped Spectrometer, may run while the array is read.
+# The newest such context is therefore kept until the next one is made (or the
+# next such one is collected, or the program ends); close() frees at once.
+_kept = []
+_made = itertools.count()
 
-    def __new__(cls, value, owner):
-        p = super().__new__(cls, value)
-        p.owner = owner
-        return p
+
+def _close_kept():
+    while True:
+        try:
+            sp = _kept.pop()
+        except IndexError:
+            return
+        sp.close()
+
+
+def _at_exit():
+    Spectrometer._keep = False
+    _close_kept()
+
+
+atexit.register(_at_exit)
 
 
 class Spectrometer:
@@ -247,10 +263,15 @@ class Spectrometer:
     ICS buffers are exposed as numpy views of the library's pinned memory.
     """
 
+    _keep = True       # False once the program is ending
+    _lent = False      # a device address was handed out
+
     def __init__(self, *, Nc, Ntpb, Nts, Nas, Np=2, Nbps=8, Npolout=None,
                  Nant=1, Nbc=0, Nb=0, Nb_host=0, gpu_index=0,
                  input_conjugated=0, incoherently_sum=0, Aws=None,
                  callback=None, record_events=True, init=True):
+        _close_kept()
+        self._serial = next(_made)
         self.ctx = RawspecContext()
         c = self.ctx
         No = len(Nts)
@@ -333,13 +354,15 @@ class Spectrometer:
         return lib().rawspec_amd_set_device_output(C.byref(self.ctx), 1 if enable else 0)
 
     def device_input(self) -> int:
-        return DevicePointer(lib().rawspec_amd_device_input(C.byref(self.ctx)) or 0, self)
+        self._lent = True
+        return lib().rawspec_amd_device_input(C.byref(self.ctx)) or 0
 
     def device_input_size(self) -> int:
         return lib().rawspec_amd_device_input_size(C.byref(self.ctx))
 
     def device_pwrbuf(self, i) -> int:
-        return DevicePointer(lib().rawspec_amd_device_pwrbuf(C.byref(self.ctx), i) or 0, self)
+        self._lent = True
+        return lib().rawspec_amd_device_pwrbuf(C.byref(self.ctx), i) or 0
 
     def stream(self) -> int:
         return lib().rawspec_amd_stream(C.byref(self.ctx)) or 0
@@ -441,6 +464,15 @@ class Spectrometer:
 
     def __del__(self):
         try:
-            self.close()
+            sp = self
+            if self._lent and self.initialized and self._keep:
+                sp = _kept.pop() if _kept else None
+                if sp is not None and sp._serial > self._serial:
+                    sp, newest = self, sp
+                else:
+                    newest = self
+                _kept.append(newest)
+            if sp is not None:
+                sp.close()
         except Exception:
             pass

@@ -1,5 +1,7 @@
-"""What a caller gets from a Spectrometer keeps the Spectrometer: its buffers
-are freed when it is collected, and a view of them read afterwards faults."""
+"""Buffers of a Spectrometer that was dropped while they are read: a numpy view
+holds it; a device address does not (an array library may keep the address for
+good), so the newest context that handed one out and was collected stays until
+the next is made, and close() frees at once."""
 import gc
 import weakref
 
@@ -11,25 +13,33 @@ import rawspec_amd as R
 class _Stub(R.Spectrometer):
     """A Spectrometer over plain host memory, without a device."""
 
-    def __init__(self):
+    def __init__(self, closed=None):
         super().__init__(Nc=1, Ntpb=8, Nts=[8], Nas=[1], init=False)
         self.mem = np.arange(64, dtype=np.float32)
-        for i in range(1):
-            self.ctx.h_pwrbuf[i] = R.C.cast(self.mem.ctypes.data, R.C.POINTER(R.C.c_float))
-            self.ctx.h_pwrbuf_size[i] = 32
+        self.closed = closed
+        self.ctx.h_pwrbuf[0] = R.C.cast(self.mem.ctypes.data, R.C.POINTER(R.C.c_float))
+        self.ctx.h_pwrbuf_size[0] = 32
+
+    def close(self):
+        if self.closed is not None:
+            self.closed.append(self._serial)
 
 
-def test_device_pointer_is_an_int_that_keeps_its_owner():
-    sp = _Stub()
-    p = R.DevicePointer(4096, sp)
-    assert p == 4096 and p + 1 == 4097 and isinstance(p, int)
-    ref = weakref.ref(sp)
-    del sp
+def test_context_with_device_addresses_outlives_its_collection():
+    closed = []
+    a, b, c = _Stub(closed), _Stub(closed), _Stub(closed)
+    for sp in (a, b):
+        sp.initialized = sp._lent = True      # as device_pwrbuf() leaves it
+    serials = [sp._serial for sp in (a, b, c)]
+    del sp, a, b, c
     gc.collect()
-    assert ref() is not None
-    del p
+    # the one that lent nothing and the older of the two are closed
+    assert sorted(closed) == [serials[0], serials[2]]
     gc.collect()
-    assert ref() is None
+    assert len(closed) == 2 and [s._serial for s in R._kept] == [serials[1]]
+    d = _Stub(closed)                         # the next context: the kept one goes
+    assert closed[-1] == serials[1] and not R._kept and len(closed) == 3
+    del d
 
 
 def test_numpy_view_keeps_its_owner():
