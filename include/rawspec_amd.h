@@ -170,7 +170,9 @@ int rawspec_amd_autotune(rawspec_context *ctx, const void *d_in, unsigned int pe
  * context's stream within each start call, so vector-bound small transforms
  * overlap memory-bound four-step passes.  Dumps and callbacks keep their
  * order on the context's stream.  rawspec_initialize() turns it on when the
- * context has both kinds of products and buffers of at least 64 MiB; a
+ * context has both kinds of products and buffers of at least 64 MiB, for
+ * calls with several buffers (on one-buffer calls the fork and join cost more
+ * than the overlap saves; once set here, it applies to every call); a
  * process running many contexts at once (more streams than hardware queues)
  * may do better with it off.  Changing it between calls is allowed.
  * rawspec_amd_set_lanes returns 0 on success; rawspec_amd_get_lanes returns

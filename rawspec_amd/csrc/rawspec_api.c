@@ -485,7 +485,7 @@ static int rs_start(rawspec_context *ctx, const void *d_in, int fft_dir)
   rs_gpu_ctx *g = rs_get(ctx);
   if (!g) return 1;
   const int fused = rsd_fused_pair(g->dev, &fa, &fb);
-  if (rsd_lanes_begin(g->dev)) return 1;
+  if (rsd_lanes_begin(g->dev, 1)) return 1;
   g->inbuf_count++;
   for (i = 0; i < ctx->No; i++) {
     int first = ((g->inbuf_count - 1) % g->Nis[i]) == 0;
@@ -526,7 +526,7 @@ static int rs_start_batch(rawspec_context *ctx, const void *const *d_in, unsigne
   if (!g) return 1;
   const int fused = rsd_fused_pair(g->dev, &fa, &fb);
   const int dumps = !g->tuning && rs_dump_queues(ctx, g);
-  if (rsd_lanes_begin(g->dev)) return 1;
+  if (rsd_lanes_begin(g->dev, nbuf)) return 1;
   for (i = 0; i < ctx->No; i++) {
     unsigned int k = 0;
     if (fused && ((int)i == fa || (int)i == fb)) {

@@ -87,9 +87,9 @@ int  rsd_run_fused(rsd_ctx *d, const void *d_in, int inverse, int first_b);
  * rsd_lane_end makes the context stream wait for product i's lane (i < 0:
  * both lanes); rsd_lane_resume makes product i's lane wait for the context
  * stream (after a dump that must precede the lane's next writes).  With
- * lanes off, or while kernel timing is on, all are no-ops and everything
+ * lanes off, in a call of one buffer (nbuf) unless the caller set the lanes, or while kernel timing is on, all are no-ops and everything
  * runs on the context stream. */
-int  rsd_lanes_begin(rsd_ctx *d);
+int  rsd_lanes_begin(rsd_ctx *d, unsigned nbuf);
 int  rsd_lane_end(rsd_ctx *d, int i);
 int  rsd_lane_resume(rsd_ctx *d, int i);
 /* Enqueues the incoherent sum of product i's integration buffer. */

@@ -268,6 +268,14 @@ struct rsd_ctx {
   hipStream_t lane[2];
   hipEvent_t ev_main, ev_lane[2];
   bool lanes;
+  // Not set by the caller: one-buffer calls stay on one stream (lanes_call: what
+  // the running call does).  Their passes are short and the fork and join per
+  // buffer cost more than the overlap saves (64 channels, 2^20, 8 and 1024
+  // points, Stokes, 128 MiB a call: 748 us on lanes, 717 on one stream; 1
+  // channel, int16, 256 MiB: 823 against 753); batches gain (the same products
+  // 8 buffers a call at level 1: 621 against 643 us a buffer, 16 channels 188
+  // against 198).
+  bool lanes_auto, lanes_call;
   rsd_config cfg;
   std::vector<float> weights;
   unsigned long long sample_bytes;     // Np * 2 * Nbps/8
@@ -324,7 +332,7 @@ static hipEvent_t ev_take(rsd_ctx *d) {
 // Lanes are used unless kernel timing is on: timed kernels run one after
 // another on the context stream, so each event pair brackets one kernel
 // running alone.
-static bool use_lanes(const rsd_ctx *d) { return d->lanes && !d->prof; }
+static bool use_lanes(const rsd_ctx *d) { return d->lanes && d->lanes_call && !d->prof; }
 
 static hipStream_t prod_stream(const rsd_ctx *d, const ProdPlan &pp) {
   return use_lanes(d) ? d->lane[pp.small ? 1 : 0] : d->stream;
@@ -882,6 +890,7 @@ static rsd_ctx *new_ctx() {
   d->lane[0] = d->lane[1] = nullptr;
   d->ev_main = d->ev_lane[0] = d->ev_lane[1] = nullptr;
   d->lanes = false;
+  d->lanes_auto = d->lanes_call = true;
   d->d_in = d->d_stage = nullptr;
   d->d_part = nullptr;
   d->d_work = d->d_tw = nullptr;
@@ -1531,7 +1540,8 @@ int rsd_tune_describe(rsd_ctx *d, int i, char *buf, size_t len) {
                   pp.fs_chunk, pp.fs_bmax);
 }
 
-int rsd_lanes_begin(rsd_ctx *d) {
+int rsd_lanes_begin(rsd_ctx *d, unsigned nbuf) {
+  d->lanes_call = nbuf > 1 || !d->lanes_auto;
   if (!use_lanes(d)) return 0;
   RSD_CHECK(hipSetDevice(d->dev));
   RSD_CHECK(hipEventRecord(d->ev_main, d->stream));
@@ -1650,6 +1660,7 @@ unsigned rsd_get_hold(rsd_ctx *d) { return d->hold_max; }
 int rsd_set_lanes(rsd_ctx *d, int enable) {
   if (enable && !(d->lane[0] && d->lane[1])) return 1;
   d->lanes = enable != 0;
+  d->lanes_auto = false;
   return 0;
 }
 
