@@ -4,18 +4,18 @@
 // the FFT-shifted sums; the reference plans these lengths with cuFFT,
 // rawspec_gpu.cu:1182-1195) for decimal lengths such as 1000 and 2000 and
 // for 3 * 2^a, which Bluestein's identity computes as two transforms of at
-// least twice the length.  A Stockham transform with mixed radices: E = 20
-// or 24 elements per thread, every stage's radix a divisor of E, so a thread
+// least twice the length.  A Stockham transform with mixed radices: E = 10,
+// 20 or 24 elements per thread, every stage's radix a divisor of E, so a thread
 // holds E / R whole butterflies of any stage and one kernel per E takes all
 // lengths of its family.  The stages' list is an argument (r_plan).
 //
-// Bound by instruction issue and LDS exchanges at 2 wavefronts per SIMD (1 for
-// E = 24 with four sums, whose sums and values are 192 registers); both
-// polarisations share an exchange, in 16-byte elements.  64 MiB of int8, 16
-// channels, two polarisations, dumps of 16 spectra of 4 sums, against Bluestein's
-// identity: 1000 points 378 -> 149 us, 2000 439 -> 136, 1536 437 -> 118, 384 383 ->
-// 141, 100 385 -> 133; one polarisation, one sum: 1000 points 233 -> 89, 1536 306
-// -> 99.
+// Bound by instruction issue and LDS exchanges, at 2 wavefronts per SIMD (E = 10:
+// 3 or 4; E = 24 with four sums, whose sums and values are 192 registers: 1);
+// both polarisations share an exchange, in 16-byte elements.  64 MiB of int8, 16
+// channels, two polarisations, dumps of 16 spectra of 4 sums, against
+// Bluestein's identity: 1000 points 378 -> 100 us, 2000 439 -> 136, 1536 437 ->
+// 118, 384 383 -> 141, 250 324 -> 91, 100 385 -> 92; one polarisation, one sum:
+// 1000 points 233 -> 77, 1536 306 -> 99.
 #include "fft_device.h"
 #include "kernels.h"
 
@@ -138,17 +138,21 @@ __device__ __forceinline__ void r_stage(float2 (&v)[NP][E], RElem<NP> *lds, cons
 template <int E, int NP, bool FIRST>
 __device__ __forceinline__ void r_pick(unsigned R, float2 (&v)[NP][E], RElem<NP> *lds, const float2 *tw, unsigned j,
                                        unsigned T, unsigned N, unsigned NS, unsigned magic) {
-  switch (R) {
-    case 2: r_stage<E, NP, 2, FIRST, false>(v, lds, tw, j, T, N, NS, magic); break;
-    case 4: r_stage<E, NP, 4, FIRST, false>(v, lds, tw, j, T, N, NS, magic); break;
-    case E / 4: r_stage<E, NP, E / 4, FIRST, false>(v, lds, tw, j, T, N, NS, magic); break;
-    case E / 2: r_stage<E, NP, E / 2, FIRST, false>(v, lds, tw, j, T, N, NS, magic); break;
-    case E: r_stage<E, NP, E, FIRST, false>(v, lds, tw, j, T, N, NS, magic); break;
-    default:
-      if constexpr (E == 24) {
-        if (R == 8) r_stage<E, NP, 8, FIRST, false>(v, lds, tw, j, T, N, NS, magic);
-        else r_stage<E, NP, 3, FIRST, false>(v, lds, tw, j, T, N, NS, magic);
-      }
+  if (R == 2) {
+    r_stage<E, NP, 2, FIRST, false>(v, lds, tw, j, T, N, NS, magic);
+  } else if (R == E / 2) {
+    r_stage<E, NP, E / 2, FIRST, false>(v, lds, tw, j, T, N, NS, magic);
+  } else if (R == E) {
+    r_stage<E, NP, E, FIRST, false>(v, lds, tw, j, T, N, NS, magic);
+  } else if constexpr (E % 4 == 0) {
+    if (R == 4) {
+      r_stage<E, NP, 4, FIRST, false>(v, lds, tw, j, T, N, NS, magic);
+    } else if (R == E / 4) {
+      r_stage<E, NP, E / 4, FIRST, false>(v, lds, tw, j, T, N, NS, magic);
+    } else if constexpr (E == 24) {
+      if (R == 8) r_stage<E, NP, 8, FIRST, false>(v, lds, tw, j, T, N, NS, magic);
+      else r_stage<E, NP, 3, FIRST, false>(v, lds, tw, j, T, N, NS, magic);
+    }
   }
 }
 
@@ -308,10 +312,12 @@ void k_small_r(SmallArgs a, RPlan rp) {
 // LDS of one slot and of the twiddles
 static unsigned r_slot_bytes(unsigned n, int np) { return (n + (n - 1) / 8) * 8u * (unsigned)np; }
 
-// The stages of an n-point transform: E = 24 for 3 * 2^a * 3^b with 8 | n, 20 for
-// 5 * 2^a * 5^b with 4 | n; as few radices (divisors of E) as make n, ascending
-// (a first stage of radix 3 or 5 writes without bank conflicts).  Slots: as many
-// spectra as 256 threads and 64 KB of LDS hold, a power of two, at most 16.
+// The stages of an n-point transform: E = 24 for 3 * 2^a * 3^b with 8 | n; for 5 *
+// 2^a * 5^b 10, or 20 where 4 | n and it takes fewer stages (1000 points as 10, 10,
+// 10 with 100 threads 100 us, as 5, 10, 20 with 50 149; 2000 as 5, 20, 20); as few
+// radices (divisors of E) as make n, ascending (a first stage of radix 3 or 5
+// writes without bank conflicts).  Slots: as many spectra as 256 threads and 64
+// KB of LDS hold, a power of two, at most 16.
 bool r_plan(unsigned n, int np, RPlan &rp) {
   if (n < kRMinN || n > 2048) return false;
   unsigned m = n;
@@ -319,36 +325,41 @@ bool r_plan(unsigned n, int np, RPlan &rp) {
   while (m % 2 == 0) m /= 2;
   if (m == 1) return false;
   while (m % P == 0) m /= P;
-  const unsigned E = P == 3 ? 24 : 20;
-  if (m != 1 || n % E) return false;
-  const unsigned div24[] = {24, 12, 8, 6, 4, 3, 2, 0}, div20[] = {20, 10, 5, 4, 2, 0};
-  const unsigned *dv = E == 24 ? div24 : div20;
-  // the last radix is E; fewest stages before it by depth-first search, larger
-  // radices first
-  unsigned best[kRMaxStages], nb = kRMaxStages, cur[kRMaxStages];
-  auto search = [&](auto &&self, unsigned left, unsigned i, unsigned from) -> void {
-    if (left == 1) {
-      nb = i;
-      for (unsigned k = 0; k < i; ++k) best[k] = cur[k];
-      return;
-    }
-    for (unsigned k = from; dv[k] && i + 1 < nb; ++k)
-      if (left % dv[k] == 0) {
-        cur[i] = dv[k];
-        self(self, left / dv[k], i + 1, k);
+  if (m != 1) return false;
+  const unsigned dv24[] = {24, 12, 8, 6, 4, 3, 2, 0}, dv20[] = {20, 10, 5, 4, 2, 0}, dv10[] = {10, 5, 2, 0};
+  const unsigned *dv[] = {P == 3 ? dv24 : dv10, P == 3 ? nullptr : dv20};
+  rp.n = kRMaxStages + 1;
+  for (int f = 0; f < 2 && dv[f]; ++f) {
+    const unsigned E = dv[f][0];
+    if (n % E) continue;
+    // the last radix is E; fewest stages before it by depth-first search, larger
+    // radices first
+    unsigned best[kRMaxStages], nb = kRMaxStages, cur[kRMaxStages];
+    auto search = [&](auto &&self, unsigned left, unsigned i, unsigned from) -> void {
+      if (left == 1) {
+        nb = i;
+        for (unsigned k = 0; k < i; ++k) best[k] = cur[k];
+        return;
       }
-  };
-  search(search, n / E, 0, 0);
-  if (nb == kRMaxStages) return false;
-  rp.e = E;
-  rp.n = nb + 1;
-  unsigned ns = 1;
-  for (unsigned i = 0; i <= nb; ++i) {
-    rp.r[i] = i < nb ? best[nb - 1 - i] : E;
-    rp.magic[i] = ((1u << 22) + ns - 1) / ns;
-    ns *= rp.r[i];
+      for (unsigned k = from; dv[f][k] && i + 1 < nb; ++k)
+        if (left % dv[f][k] == 0) {
+          cur[i] = dv[f][k];
+          self(self, left / dv[f][k], i + 1, k);
+        }
+    };
+    search(search, n / E, 0, 0);
+    if (nb == kRMaxStages || nb + 1 >= rp.n) continue;
+    rp.e = E;
+    rp.n = nb + 1;
+    unsigned ns = 1;
+    for (unsigned i = 0; i <= nb; ++i) {
+      rp.r[i] = i < nb ? best[nb - 1 - i] : E;
+      rp.magic[i] = ((1u << 22) + ns - 1) / ns;
+      ns *= rp.r[i];
+    }
   }
-  const unsigned t = n / E;
+  if (rp.n > kRMaxStages) return false;
+  const unsigned t = n / rp.e;
   rp.slots = 1;
   while (rp.slots < 16 && 2 * rp.slots * t <= 256 && 2 * rp.slots * r_slot_bytes(n, np) + 8 * n <= 65536) rp.slots *= 2;
   rp.threads = (rp.slots * t + 63) / 64 * 64;
@@ -375,9 +386,11 @@ int launch_small_r(int nbps, int np, int pmode, const SmallArgs &a, const RPlan 
     return 2;
   const unsigned lds = rp.slots * r_slot_bytes(a.nt, np) + 8 * a.nt;
   if (nbps == 8)
-    return rp.e == 24 ? go_r<24, 8>(np, pmode, a, rp, nblocks, lds, s) : go_r<20, 8>(np, pmode, a, rp, nblocks, lds, s);
+    return rp.e == 24 ? go_r<24, 8>(np, pmode, a, rp, nblocks, lds, s)
+         : rp.e == 20 ? go_r<20, 8>(np, pmode, a, rp, nblocks, lds, s) : go_r<10, 8>(np, pmode, a, rp, nblocks, lds, s);
   if (nbps == 16)
-    return rp.e == 24 ? go_r<24, 16>(np, pmode, a, rp, nblocks, lds, s) : go_r<20, 16>(np, pmode, a, rp, nblocks, lds, s);
+    return rp.e == 24 ? go_r<24, 16>(np, pmode, a, rp, nblocks, lds, s)
+         : rp.e == 20 ? go_r<20, 16>(np, pmode, a, rp, nblocks, lds, s) : go_r<10, 16>(np, pmode, a, rp, nblocks, lds, s);
   return 2;
 }
 

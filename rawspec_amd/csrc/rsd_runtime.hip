@@ -716,14 +716,13 @@ static bool f8_on(const rsd_ctx *d) { return d->f8_a >= 0 && d->mfma == 1; }
 // Bluestein's: nearly always, but a buffer of few points waits for the chain of
 // one transform, which more threads with less work each make shorter (4
 // channels, 1152 points, dumps of 8 spectra of 4 sums: 1 MiB 29 against 18 us,
-// 4 MiB 34 against 61, 32 MiB 95 against 298; one sum 18 against 16, 21 against
-// 35, 74 against 187; 2000 points, one sum: 14 against 16, 17 against 22, 68
-// against 157).  The lines are 2^18 points of one polarisation, 2^19 of two,
-// 2^20 of two with four sums.  Four sums of the shortest lengths leave too many
-// sums to write (48 points 267 against 216 us, 80 points 120 against 485).
+// 2 MiB 31 against 33, 32 MiB 95 against 298; one sum 18 against 16, 18 against
+// 20, 74 against 187).  The line is at 2 MiB of int8, 2^18 points a polarisation.
+// Four sums of the shortest lengths leave too many sums to write (48 points 267
+// against 216 us, 80 points 120 against 485).
 static bool r_pays(const rsd_config *cfg, const ProdPlan &pp) {
   const unsigned long long points = (unsigned long long)cfg->Nc * pp.p.Nss * pp.p.Nt;
-  return points >= (1ull << 17) * cfg->Np * (pp.Q == 1 ? 2 : 4) && pp.p.Nt >= (pp.Q == 1 ? 40u : 80u);
+  return points >= (1ull << 18) * cfg->Np && pp.p.Nt >= (pp.Q == 1 ? 40u : 80u);
 }
 
 static int plan_all(const rsd_config *cfg, rsd_ctx *d) {

@@ -3,8 +3,7 @@ lengths the reference plans with cuFFT, rawspec_gpu.cu:1182-1195), against the
 FP64 oracle at the FP32 bar of the other lengths.  A transform of N points
 rounds about log2 N times, as Bluestein's and the power-of-two kernels do, so
 their tolerance holds unchanged.  Each buffer holds enough points for this
-kernel to take the product (2^20 with two polarisations and four sums, 2^19
-with one, 2^18 of one polarisation); the lengths take every radix of both
+kernel to take the product (2^18 a polarisation); the lengths take every radix of all
 families first, in the middle and last, workgroups of 1 to 16 spectra that
 are not full wavefronts, dumps of one spectrum (sums from registers), of a few,
 and split over workgroups.
@@ -16,7 +15,7 @@ from tests.spectro_cases import PLAIN_TOL, check_results, run_case
 pytestmark = pytest.mark.gpu
 
 CASES = {
-    # stages 5,20,20 / 5,10,20 / 20,20: one and several spectra per workgroup
+    # stages 5,20,20 / 10,10,10 / 20,20: one and several spectra per workgroup
     "2000_stokes": dict(Nc=4, Ntpb=2000 * 136, Nts=[2000, 1000, 400], Nas=[1, 34, 680], Npolout=[-4, -4, -4]),
     # 4,20,20 / 2,20,20 / 4,20
     "1600_full_int16": dict(Nc=3, Ntpb=1600 * 220, Nts=[1600, 800, 80], Nas=[20, 440, 2], Npolout=[4, 1, 4], Nbps=16),
@@ -30,7 +29,9 @@ CASES = {
     # 3,24,24 / 3,12,24 / 12,24 / 6,24 with four sums
     "1728_full_inverse": dict(Nc=6, Ntpb=1728 * 104, Nts=[1728, 864, 288, 144], Nas=[8, 208, 16, 1], Npolout=[4, -4, 4, -4],
                               fft_dir=-1),
-    # 5,5,20 / 5,20 / 10,20 of one polarisation, integrated over two buffers
+    # 5,5,5,10 / 5,5,10 / 5,10
+    "1250_stokes": dict(Nc=6, Ntpb=1250 * 160, Nts=[1250, 250, 50], Nas=[16, 1, 1000], Npolout=[-4, 4, 1]),
+    # 10,10,10 / 5,10,10 / 10,10 / 10,20 of one polarisation, integrated over two buffers
     "500_one_pol": dict(Nc=3, Ntpb=1000 * 96, Nts=[1000, 500, 100, 200], Nas=[192, 4, 960, 1], Npolout=[1] * 4, Np=1),
 }
 
