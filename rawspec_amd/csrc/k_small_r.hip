@@ -157,7 +157,7 @@ __device__ __forceinline__ void r_pick(unsigned R, float2 (&v)[NP][E], RElem<NP>
 }
 
 template <int E, int NBPS, int NP, int PMODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(E == 24 && PMODE != 1 ? 1 : 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(E > 10 && PMODE != 1 ? 1 : 2)))
 void k_small_r(SmallArgs a, RPlan rp) {
   constexpr int Q = nq<PMODE>();
   using S = Sample<NBPS, NP>;
@@ -313,12 +313,14 @@ void k_small_r(SmallArgs a, RPlan rp) {
 static unsigned r_slot_bytes(unsigned n, int np) { return (n + (n - 1) / 8) * 8u * (unsigned)np; }
 
 // The stages of an n-point transform: E = 24 for 3 * 2^a * 3^b with 8 | n; for 5 *
-// 2^a * 5^b 10, or 20 where 4 | n and it takes fewer stages (1000 points as 10, 10,
+// 2^a * 5^b 10, or 20 where 4 | n and it takes fewer stages, for four sums
+// only where 10 does not make n (20 would hold 160 registers of values and sums: 1
+// wavefront per SIMD) (1000 points as 10, 10,
 // 10 with 100 threads 100 us, as 5, 10, 20 with 50 149; 2000 as 5, 20, 20); as few
 // radices (divisors of E) as make n, ascending (a first stage of radix 3 or 5
 // writes without bank conflicts).  Slots: as many spectra as 256 threads and 64
 // KB of LDS hold, a power of two, at most 16.
-bool r_plan(unsigned n, int np, RPlan &rp) {
+bool r_plan(unsigned n, int np, int pmode, RPlan &rp) {
   if (n < kRMinN || n > 2048) return false;
   unsigned m = n;
   const unsigned P = n % 3 == 0 ? 3 : 5;
@@ -331,7 +333,7 @@ bool r_plan(unsigned n, int np, RPlan &rp) {
   rp.n = kRMaxStages + 1;
   for (int f = 0; f < 2 && dv[f]; ++f) {
     const unsigned E = dv[f][0];
-    if (n % E) continue;
+    if (n % E || (f == 1 && pmode != 1 && rp.n <= kRMaxStages)) continue;
     // the last radix is E; fewest stages before it by depth-first search, larger
     // radices first
     unsigned best[kRMaxStages], nb = kRMaxStages, cur[kRMaxStages];
@@ -381,7 +383,7 @@ int launch_small_r(int nbps, int np, int pmode, const SmallArgs &a, const RPlan 
                    hipStream_t s) {
   if (nblocks == 0) return 0;
   RPlan w;
-  if (!r_plan(a.nt, np, w) || w.e != rp.e || w.slots != rp.slots || w.threads != rp.threads || w.n != rp.n ||
+  if (!r_plan(a.nt, np, pmode, w) || w.e != rp.e || w.slots != rp.slots || w.threads != rp.threads || w.n != rp.n ||
       a.spg * a.gpw != rp.slots || !a.chirp || (np != 1 && np != 2))
     return 2;
   const unsigned lds = rp.slots * r_slot_bytes(a.nt, np) + 8 * a.nt;

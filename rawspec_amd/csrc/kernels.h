@@ -160,7 +160,7 @@ int launch_small_h(int n, int nbps, int np, int pmode, const SmallArgs &a, unsig
                    int waves, hipStream_t s);
 // Lengths 2^a 3^b and 2^a 5^b (k_small_r.hip): r_plan fills rp, or returns false
 // where the length is Bluestein's; a.chirp holds W_N^n.
-bool r_plan(unsigned n, int np, RPlan &rp);
+bool r_plan(unsigned n, int np, int pmode, RPlan &rp);
 int launch_small_r(int nbps, int np, int pmode, const SmallArgs &a, const RPlan &rp, unsigned nblocks,
                    hipStream_t s);
 // Matrix-core fused small kernel (N = 1024, two pols): one wavefront per

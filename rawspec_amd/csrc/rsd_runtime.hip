@@ -450,6 +450,15 @@ static void plan_small_h(rsd_ctx *d, ProdPlan &pp) {
   pp.h_bpc = 1;
   pp.h_waves = 4;
   const unsigned long long groups = (unsigned long long)Nc * pp.Ng;
+  // Few groups of two or three units: a wavefront takes its units in turn, where
+  // the vector kernel spreads them over a workgroup (55 groups of 3 spectra of
+  // 1024 points, int16 power: 14.3 against 6.8 us, int8 Stokes 10.9 against 9.9;
+  // 1024 groups of int8 12.3 against 14.0, 14.1 against 25.2).  Two units with
+  // four sums are even at 16 groups and better beyond.
+  if ((upg == 3 || (upg == 2 && pp.Q == 1)) && groups < (pp.Q == 1 ? 513u : 512u)) {
+    pp.h_ok = 0;
+    return;
+  }
   pp.h_solo = groups >= kHybSoloWaves || upg < 4;
   if (pp.h_solo) {
     // at most 8 wavefronts per SIMD's two slots, so that the last round is short
@@ -610,7 +619,9 @@ static unsigned fs_chunk_for(const rsd_ctx *d, const ProdPlan &pp, unsigned kb) 
 // 32 workgroups, each summing thousands of spectra.  A split pays while the
 // (k2 tile, group, channel) workgroups of all Nc channels are fewer than
 // kFsbFull per 2 CUs: at 1.5 per CU and more it gained nothing (2^17 points,
-// 32 spectra, 12 channels 0.9..1.05x), at one 1.1..1.24x.  Runs cost a launch and
+// 32 spectra, 12 channels 0.9..1.05x), at one 1.1..1.24x; workgroups of one
+// polarisation hold half the registers, so twice as many run together (2^20
+// points, 2 channels, 128 spectra, two per CU: 700 us whole, 470 split).  Runs cost a launch and
 // their partial sums' traffic, which grows with their number, as their gain
 // shrinks: the time n t / ns + ns c is least at ns^2 = n t / c, about n
 // kFsbRunSums / (sums of the launch); twice and four times that lost up to
@@ -621,10 +632,10 @@ static unsigned fs_chunk_for(const rsd_ctx *d, const ProdPlan &pp, unsigned kb) 
 // context's channels, not on a launch's channel chunk, so every path over the
 // same buffers (batched, held, allocation-free with its smaller chunks) adds
 // the same runs in the same order.
-static unsigned fsb_runs(const ProdPlan &pp, unsigned cus, unsigned Nc, unsigned na_buf) {
+static unsigned fsb_runs(const ProdPlan &pp, unsigned cus, unsigned Nc, unsigned Np, unsigned na_buf) {
   const unsigned long long base =
       (unsigned long long)(pp.N2 / (unsigned)rsk::fs_tile_b((int)pp.N1)) * pp.Ng * Nc;
-  if (base == 0 || 2 * base >= (unsigned long long)cus * kFsbFull) return 1;
+  if (base == 0 || 2 * base >= (unsigned long long)cus * (Np == 1 ? 2 * kFsbWgPerCu : kFsbFull)) return 1;
   unsigned long long ns = ((unsigned long long)cus * kFsbWgPerCu + base - 1) / base;
   if (ns > na_buf) ns = na_buf;
   const unsigned long long sums = (unsigned long long)pp.Q * pp.p.Nt * pp.Ng * Nc;
@@ -648,7 +659,7 @@ static size_t fsb_part_need(const rsd_ctx *d, const ProdPlan &pp) {
   if (pp.small) return 0;
   const unsigned kb = pp.p.Nis < (unsigned)rsk::kMaxBatch ? pp.p.Nis : (unsigned)rsk::kMaxBatch;
   const unsigned na = (kb > 1 ? kb : 1) * pp.na_buf;
-  return fsb_part_floats(pp, fsb_runs(pp, kPlanCus, d->cfg.Nc, na), d->cfg.Nc);
+  return fsb_part_floats(pp, fsb_runs(pp, kPlanCus, d->cfg.Nc, d->cfg.Np, na), d->cfg.Nc);
 }
 
 // Launch plan of one product from its tunables; returns the float2
@@ -758,7 +769,7 @@ static int plan_all(const rsd_config *cfg, rsd_ctx *d) {
     if (pp.bs) {
       pp.bs_m = 1;
       while (pp.bs_m < 2 * N - 1) pp.bs_m <<= 1;
-      pp.r_ok = r_pays(cfg, pp) && rsk::r_plan(N, (int)cfg->Np, pp.rp);
+      pp.r_ok = r_pays(cfg, pp) && rsk::r_plan(N, (int)cfg->Np, pp.p.npolout, pp.rp);
     }
     pp.small = pp.bs || N <= (unsigned)rsk::kTwN;
     pp.t_target = 2048;
@@ -1206,7 +1217,7 @@ static int launch_pass_b(rsd_ctx *d, int i, rsk::FsArgs a, hipStream_t s) {
   }
   // split the dump groups into runs where the launch is too narrow for the
   // GPU, as far as the partial-sum buffer allows
-  unsigned ns = fsb_runs(pp, d->cus < kPlanCus ? d->cus : kPlanCus, d->cfg.Nc, a.na_buf);
+  unsigned ns = fsb_runs(pp, d->cus < kPlanCus ? d->cus : kPlanCus, d->cfg.Nc, d->cfg.Np, a.na_buf);
   const size_t per_run = fsb_part_floats(pp, 2, a.nch) / 2;
   if (ns > 1 && per_run && (size_t)ns * per_run > d->partb_len) ns = (unsigned)(d->partb_len / per_run);
   if (ns > 1) {
