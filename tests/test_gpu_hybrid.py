@@ -105,3 +105,13 @@ def test_fourstep_first_pass(lg, np_, bits):
         print(f"case: {kw}", flush=True)
         res, cfg = run_device_case(**kw)
         check_results(res, cfg, tol_by_product={0: 1e-3, 1: 1e-3} if level else None)
+
+
+@pytest.mark.parametrize("np_, mode", [(1, 1), (2, 1), (2, -4)])
+@pytest.mark.parametrize("nt", [1, 2, 4, 8, 16, 32, 2048, 4096])
+def test_int8_lengths_in_fp16_up_to_the_first_exchange(nt, np_, mode):
+    # the vector kernel's int8 lengths: whole groups, one spectrum per dump
+    s = 8192 * 3
+    for fwd in (True, False):
+        assert run(Nc=2, Ntpb=s, Nts=[nt, nt], Nas=[s // nt // 3, 1], Np=np_, bits=8,
+                   pols=[mode] * 2, fwd=fwd, conj=0) <= PLAIN_TOL
