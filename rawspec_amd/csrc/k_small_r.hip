@@ -13,7 +13,7 @@
 // 3 or 4; E = 24 with four sums, whose sums and values are 192 registers: 1);
 // both polarisations share an exchange, in 16-byte elements.  64 MiB of int8, 16
 // channels, two polarisations, dumps of 16 spectra of 4 sums, against
-// Bluestein's identity: 1000 points 378 -> 100 us, 2000 439 -> 136, 1536 437 ->
+// Bluestein's identity: 1000 points 378 -> 100 us, 2000 439 -> 123, 1536 437 ->
 // 118, 384 383 -> 141, 250 324 -> 91, 100 385 -> 92; one polarisation, one sum:
 // 1000 points 233 -> 77, 1536 306 -> 99.
 #include "fft_device.h"
