@@ -417,19 +417,21 @@ int launch_fs_b(int np, int pmode, const FsArgs &a, hipStream_t s) {
   return 2;
 }
 
-// One thread per four values of the launch's sums: the ns partial sums in run
+// One thread per V values of the launch's sums: the ns partial sums in run
 // order, then the finish k_fs_b applies to its own sums (same scale, same
 // internal-accumulator block, same shifted output position).  Bound by the
 // partial sums' bytes: 16-byte loads, four runs in flight, and shifts for the
 // power-of-two sizes (single floats placed by 64-bit divisions took 28 us for
-// four runs of 2^18 points x 3 x 4 sums, 50 MB).
-template <int Q>
+// four runs of 2^18 points x 3 x 4 sums, 50 MB).  The V values are consecutive
+// k2 of one k1, so V is at most pass B's tile: 4, or the 2 and 1 columns of
+// N1 = 2048 and 4096.
+template <int Q, int V>
 __global__ __launch_bounds__(256) void k_fs_b_reduce(FsArgs a, unsigned lTB) {
-  using f4 = float __attribute__((ext_vector_type(4)));
+  using fv = float __attribute__((ext_vector_type(V)));
   const unsigned N1 = a.N1, N2 = a.N2, lN1 = 31 - __builtin_clz(N1), TB = 1u << lTB;
   const unsigned long long N = (unsigned long long)N1 * N2;
   // idx runs over [tiles][Q][N1][TB], one (group, channel)'s block of a run
-  const unsigned idx = (blockIdx.x * 256 + threadIdx.x) * 4;
+  const unsigned idx = (blockIdx.x * 256 + threadIdx.x) * V;
   const unsigned sg = idx & (TB - 1), k1 = (idx >> lTB) & (N1 - 1);
   const unsigned tq = idx >> (lTB + lN1), q = tq % Q, tile = tq / Q;
   const unsigned rows = a.Ng * a.nch;
@@ -437,41 +439,47 @@ __global__ __launch_bounds__(256) void k_fs_b_reduce(FsArgs a, unsigned lTB) {
   for (unsigned gc = blockIdx.y; gc < rows; gc += gridDim.y) {
     const unsigned g = gc / a.nch, c = a.c0 + (gc - g * a.nch);
     const float *p = a.partb + (unsigned long long)gc * Q * N + idx;
-    f4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    fv sum = 0.0f;
     for (unsigned run = 0; run < a.ns; run += 4) {
-      f4 v[4];
+      fv v[4];
 #pragma unroll
       for (unsigned u = 0; u < 4; ++u)
-        if (run + u < a.ns) v[u] = *reinterpret_cast<const f4 *>(p + (run + u) * total);
+        if (run + u < a.ns) v[u] = *reinterpret_cast<const fv *>(p + (run + u) * total);
 #pragma unroll
       for (unsigned u = 0; u < 4; ++u)
         if (run + u < a.ns) sum += v[u];
     }
-    f4 v = sum * a.scale;
-    f4 *ie = reinterpret_cast<f4 *>(a.acc_int + (((unsigned long long)g * a.Nc + c) * Q * N + idx));
+    fv v = sum * a.scale;
+    fv *ie = reinterpret_cast<fv *>(a.acc_int + (((unsigned long long)g * a.Nc + c) * Q * N + idx));
     if (a.mode == FS_MID || a.mode == FS_LAST) v += *ie;
     if (a.mode == FS_FIRST || a.mode == FS_MID) {
       *ie = v;
     } else {
       float *o = a.acc + (((unsigned long long)g * Q + q) * a.Nc + c) * N + tile * TB + sg +
                  (unsigned long long)N2 * ((k1 + N1 / 2) & (N1 - 1));
-      *reinterpret_cast<f4 *>(o) = v;
+      *reinterpret_cast<fv *>(o) = v;
     }
   }
+}
+
+template <int V>
+static int go_reduce(unsigned Q, const FsArgs &a, hipStream_t s) {
+  const unsigned long long rows = (unsigned long long)a.Ng * a.nch;
+  const unsigned nb = a.N1 * a.N2 / (256 * V) * Q;    // N1, N2 >= 64
+  if (rows == 0 || rows > 0xffffffffull || nb == 0) return 2;
+  const dim3 grid(nb, rows < 65535 ? (unsigned)rows : 65535u);
+  const unsigned lTB = (unsigned)__builtin_ctz((unsigned)fs_tile_b((int)a.N1));
+  if (Q == 1) hipLaunchKernelGGL((k_fs_b_reduce<1, V>), grid, dim3(256), 0, s, a, lTB);
+  else hipLaunchKernelGGL((k_fs_b_reduce<4, V>), grid, dim3(256), 0, s, a, lTB);
+  return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
 int launch_fs_b_reduce(int pmode, const FsArgs &a, hipStream_t s) {
   if (a.ns < 2 || !runs_ok(a)) return 2;
   const unsigned Q = pmode == 1 ? 1u : 4u;
   const unsigned TB = (unsigned)fs_tile_b((int)a.N1);
-  const unsigned long long rows = (unsigned long long)a.Ng * a.nch;
-  const unsigned nb = a.N1 * a.N2 / 1024 * Q;    // N1, N2 >= 64
-  if (rows == 0 || rows > 0xffffffffull || nb == 0) return 2;
-  const dim3 grid(nb, rows < 65535 ? (unsigned)rows : 65535u);
-  const unsigned lTB = (unsigned)__builtin_ctz(TB);
-  if (Q == 1) hipLaunchKernelGGL((k_fs_b_reduce<1>), grid, dim3(256), 0, s, a, lTB);
-  else hipLaunchKernelGGL((k_fs_b_reduce<4>), grid, dim3(256), 0, s, a, lTB);
-  return hipGetLastError() == hipSuccess ? 0 : 1;
+  if (TB >= 4) return go_reduce<4>(Q, a, s);
+  return TB == 2 ? go_reduce<2>(Q, a, s) : go_reduce<1>(Q, a, s);
 }
 
 }  // namespace rsk
