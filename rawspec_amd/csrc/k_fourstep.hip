@@ -417,8 +417,9 @@ int launch_fs_b(int np, int pmode, const FsArgs &a, hipStream_t s) {
   return 2;
 }
 
-// One thread per V values of the launch's sums: the ns partial sums in run
-// order, then the finish k_fs_b applies to its own sums (same scale, same
+// One thread per V values of the launch's sums: the ns partial sums in four
+// running sums (one over all would round ns times in turn; up to 128 runs of
+// single spectra), then the finish k_fs_b applies to its own sums (same scale, same
 // internal-accumulator block, same shifted output position).  Bound by the
 // partial sums' bytes: 16-byte loads, four runs in flight, and shifts for the
 // power-of-two sizes (single floats placed by 64-bit divisions took 28 us for
@@ -439,7 +440,7 @@ __global__ __launch_bounds__(256) void k_fs_b_reduce(FsArgs a, unsigned lTB) {
   for (unsigned gc = blockIdx.y; gc < rows; gc += gridDim.y) {
     const unsigned g = gc / a.nch, c = a.c0 + (gc - g * a.nch);
     const float *p = a.partb + (unsigned long long)gc * Q * N + idx;
-    fv sum = 0.0f;
+    fv s[4] = {};
     for (unsigned run = 0; run < a.ns; run += 4) {
       fv v[4];
 #pragma unroll
@@ -447,8 +448,9 @@ __global__ __launch_bounds__(256) void k_fs_b_reduce(FsArgs a, unsigned lTB) {
         if (run + u < a.ns) v[u] = *reinterpret_cast<const fv *>(p + (run + u) * total);
 #pragma unroll
       for (unsigned u = 0; u < 4; ++u)
-        if (run + u < a.ns) sum += v[u];
+        if (run + u < a.ns) s[u] += v[u];
     }
+    const fv sum = (s[0] + s[1]) + (s[2] + s[3]);
     fv v = sum * a.scale;
     fv *ie = reinterpret_cast<fv *>(a.acc_int + (((unsigned long long)g * a.Nc + c) * Q * N + idx));
     if (a.mode == FS_MID || a.mode == FS_LAST) v += *ie;

@@ -25,18 +25,19 @@ __global__ __launch_bounds__(256) void k_reduce(ReduceArgs a) {
     const unsigned c = (unsigned)(r / a.Ng);
     const float *p = a.part + ((((unsigned long long)c * a.Ng + g) * a.G) * a.Q + q) * a.N + jo;
     const unsigned long long step = (unsigned long long)a.Q * a.N;
-    // partials in order, eight loads in flight: a launch of few outputs is
-    // bound by the chain of loads (64 partials of 65536 outputs: 42 to 12 us)
-    float sum = 0.0f;
-    unsigned ch = 0;
-    for (; ch + 8 <= a.G; ch += 8) {
+    // Eight loads in flight: a launch of few outputs is bound by the chain of
+    // loads (64 partials of 65536 outputs: 42 to 12 us).  Eight running sums,
+    // joined pairwise, in a fixed order: one over all partials would round G
+    // times in turn.
+    float s[8] = {};
+    for (unsigned ch = 0; ch < a.G; ch += 8) {
       float v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = p[(ch + u) * step];
+      for (unsigned u = 0; u < 8; ++u) v[u] = ch + u < a.G ? p[(ch + u) * step] : 0.0f;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) sum += v[u];
+      for (int u = 0; u < 8; ++u) s[u] += v[u];
     }
-    for (; ch < a.G; ++ch) sum += p[ch * step];
+    const float sum = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
     float *o = a.acc + (((unsigned long long)g * a.Q + q) * a.Nc + c) * a.N + jo;
     const float val = sum * a.scale;
     *o = a.first ? val : (*o + val);

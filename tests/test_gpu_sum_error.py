@@ -18,6 +18,11 @@ TOL = 1.5e-7
 CASES = {
     # pass B over 32 spectra in one run: 32 terms, not the 128 products
     "2^17 two pols": (1 << 17, 32, 1, 12, 2, 8),
+    # 128 runs of single spectra, added by k_fs_b_reduce
+    "8192 one pol": (8192, 128, 1, 1, 1, 8),
+    "8192 two pols": (8192, 128, 1, 1, 2, 8),
+    # 256 partial sums of 4 spectra, added by k_reduce
+    "1024 one channel": (1024, 1024, 1, 1, 2, 8),
 }
 
 
