@@ -17,7 +17,8 @@
 //   SOLO   every wavefront integrates whole groups, one after another, and
 //          stores each from registers (many short groups);
 //   else   the workgroup's wavefronts share one chunk of a group and add
-//          their sums through LDS in wavefront order (few long groups).
+//          their sums through LDS in wavefront order (few groups, or long ones,
+//          whose chains of FP32 additions would round more in one wavefront).
 #include <type_traits>
 
 #include "dft_hybrid.h"
@@ -28,7 +29,7 @@ namespace rsk {
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 template <int N, int NBPS, int NP, int PMODE, bool SOLO, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, PMODE == 1 && !(NBPS == 16 && NP == 2 && N == 256) ? 3 : 2) void k_small_h(SmallArgs a) {
+__global__ __launch_bounds__(64 * WAVES, PMODE == 1 ? 3 : 2) void k_small_h(SmallArgs a) {
   constexpr int M = N / 32, S = 1024 / N;
   constexpr int Q = nq<PMODE>();
   constexpr int AC = M <= 16 ? M : 16;         // bins per lane while integrating
@@ -101,6 +102,27 @@ __global__ __launch_bounds__(64 * WAVES, PMODE == 1 && !(NBPS == 16 && NP == 2 &
   const float gam = a.gam * a.isign;
   const float sc = a.scale * (In::SCALE * In::SCALE);
 
+  // The unit's spectra of a bin are added up before they join the running sum (a
+  // single spectrum's four sums are not: an eighth more instructions)
+  auto sum_unit = [&](const float2 (&x0)[16], const float2 (&x1)[16]) {
+#pragma unroll
+    for (int d = 0; d < AC; ++d) {
+      if constexpr (PMODE == 1) {              // one pol
+        float t = fmaf(x0[d].y, x0[d].y, x0[d].x * x0[d].x);
+#pragma unroll
+        for (int r = d + AC; r < 16; r += AC) t += fmaf(x0[r].y, x0[r].y, x0[r].x * x0[r].x);
+        acc[d][0] += t;
+      } else if constexpr (AC == 16) {
+        detect_raw_np<PMODE, NP>(acc[d], x0[d], x1[d]);
+      } else {
+        float t[Q] = {};
+#pragma unroll
+        for (int r = d; r < 16; r += AC) detect_raw_np<PMODE, NP>(t, x0[r], x1[r]);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) acc[d][q] += t[q];
+      }
+    }
+  };
   u32x4 ahead[VL];                             // the next unit's samples
   if (nu) {
 #pragma unroll
@@ -148,9 +170,7 @@ __global__ __launch_bounds__(64 * WAVES, PMODE == 1 && !(NBPS == 16 && NP == 2 &
       dft32_mfma<1, In::PARTS>(f, K, lane + z, r1, i1);
       if constexpr (PMODE == 1) {
         hyb_stage2<M>(r1[0], i1[0], tg, x[0]);
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[r & (AC - 1)][0] = fmaf(x[0][r].y, x[0][r].y, fmaf(x[0][r].x, x[0][r].x, acc[r & (AC - 1)][0]));
+        sum_unit(x[0], x[0]);
       } else {
         zr[p] = r1[0];
         zi[p] = i1[0];
@@ -169,8 +189,7 @@ __global__ __launch_bounds__(64 * WAVES, PMODE == 1 && !(NBPS == 16 && NP == 2 &
     if constexpr (PMODE != 1) {
 #pragma unroll
       for (int p = 0; p < NP; ++p) hyb_stage2<M>(zr[p], zi[p], tg, x[p]);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) detect_raw_np<PMODE, NP>(acc[r & (AC - 1)], x[0][r], x[NP - 1][r]);
+      sum_unit(x[0], x[NP - 1]);
     }
 
     if constexpr (SOLO) {
@@ -259,12 +278,27 @@ __global__ __launch_bounds__(64 * WAVES, PMODE == 1 && !(NBPS == 16 && NP == 2 &
   }
 }
 
+// int16 products that the planner never sends here (rsd_runtime.hip, vector_pays):
+// 64 points; power of two pols at 256 points, and from 256 points on where
+// wavefronts take whole groups.
+template <int N, int NBPS, int NP, int PMODE, bool SOLO>
+constexpr bool h_built() {
+  return NBPS == 8 || !(N == 64 || (N >= 256 && PMODE == 1 && (SOLO || (N == 256 && NP == 2))));
+}
 template <int N, int NBPS, int NP, int PMODE>
 static int go_h(const SmallArgs &a, unsigned nb, int solo, int waves, hipStream_t s) {
   const dim3 g(nb), t(64 * waves);
-  if (solo) hipLaunchKernelGGL((k_small_h<N, NBPS, NP, PMODE, true, 4>), g, t, 0, s, a);
-  else if (waves == 8) hipLaunchKernelGGL((k_small_h<N, NBPS, NP, PMODE, false, 8>), g, t, 0, s, a);
-  else hipLaunchKernelGGL((k_small_h<N, NBPS, NP, PMODE, false, 4>), g, t, 0, s, a);
+  if (solo) {
+    if constexpr (h_built<N, NBPS, NP, PMODE, true>())
+      hipLaunchKernelGGL((k_small_h<N, NBPS, NP, PMODE, true, 4>), g, t, 0, s, a);
+    else return 2;
+  } else if constexpr (!h_built<N, NBPS, NP, PMODE, false>()) {
+    return 2;
+  } else if (waves == 8) {
+    hipLaunchKernelGGL((k_small_h<N, NBPS, NP, PMODE, false, 8>), g, t, 0, s, a);
+  } else {
+    hipLaunchKernelGGL((k_small_h<N, NBPS, NP, PMODE, false, 4>), g, t, 0, s, a);
+  }
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 

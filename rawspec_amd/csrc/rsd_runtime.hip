@@ -374,8 +374,11 @@ static void plan_small(rsd_ctx *d, ProdPlan &pp) {
   // per slot.  From 2048 points a workgroup's one or two slots hold a CU's
   // registers for two workgroups: 512 of them fill it, and more only write
   // partial sums (4096 points, Stokes, 64 MiB in dumps of 4 spectra: 67
-  // against 141 us).
-  const unsigned long long target = n >= 2048 ? pp.t_target / 4 : pp.t_target;
+  // against 141 us).  So do the mixed-radix kernel's beyond 512 points (768
+  // points, 8 MiB of Stokes 45 against 94 us, of power 39 against 57; 250 points
+  // 44 against 50 and 38 against 35, 48 points 31 against 31 and 21 against 16).
+  const bool few = pp.r_ok ? pp.p.Nt > 512 : n >= 2048;
+  const unsigned long long target = few ? pp.t_target / 4 : pp.t_target;
   while ((unsigned long long)Nc * pp.Ng * (pp.na_buf / pp.chunk) < target && pp.chunk % 2 == 0 &&
          pp.chunk / 2 >= (slots > vslots ? slots : vslots))
     pp.chunk /= 2;
@@ -430,36 +433,68 @@ static void plan_small_mfma(rsd_ctx *d, ProdPlan &pp) {
 
 // Plan of the small kernel whose first 32 points run on the matrix cores
 // (k_small_h.hip).  Where the channels' groups alone make kHybSoloWaves
-// wavefronts, each wavefront integrates whole groups; otherwise the groups
+// wavefronts, each wavefront integrates whole groups of up to kHybSoloUnits
+// units of 1024 samples; longer groups are shared by a workgroup's 4 wavefronts,
+// whose shorter chains of additions round less, at the same speed (error and
+// speed over the vector kernel's at 256 MiB: 8 units at most 1.07, 12 units 1.12
+// whole and 1.04 shared, 32 units 1.36 and 1.04; 1024 points, 12 units, Stokes
+// 1.45 times as fast whole and 1.37 shared, power 1.28 and 1.38).  Fewer groups
 // are halved into chunks until t_target / 4 workgroups are busy (default 512,
-// two per CU: 1024 read 64 MiB no faster and wrote twice the partial sums),
-// each of a chunk's 4 wavefronts keeping a unit of 1024 samples.
-constexpr unsigned kHybSoloWaves = 2048;
+// two per CU: 1024 read 64 MiB no faster and wrote twice the partial sums), each
+// of a chunk's 4 wavefronts keeping a unit; beyond that up to t_target, as the
+// vector kernel's, where chunks are longer than kHybChunkUnits (512 groups of 256
+// units whole: 1.04 to 1.22 times the vector kernel's error, 0.7 to 1.4 times its
+// speed).
+constexpr unsigned kHybSoloWaves = 2048, kHybSoloUnits = 8, kHybChunkUnits = 64;
+// Groups for which the vector kernel, with a workgroup each, has all of them
+// resident (two per CU).
+constexpr unsigned kVecResident = 512;
+
+// Whether the vector kernel is the better one for groups of upg units.  Figures:
+// the hybrid kernel's speed over the vector kernel's.
+// - Single spectra of 1024 points: wavefronts store as much as they read and
+//   nothing hides it (0.5 to 1.0).
+// - Groups of two or three units, all resident: a wavefront takes its units in
+//   turn, where the vector kernel spreads them over a workgroup (power of two
+//   units: 512 groups 0.82, 640 groups 1.04; of three 0.80, 0.95, 1024 groups 1.1;
+//   Stokes of three: 256 groups 0.92, 512 1.13, 640 1.57; Stokes of two 1.1 to 1.9).
+// - int16 takes twice the matrix instructions and operands.  64 points: 0.73 to 1.0
+//   (Stokes of one unit 1.25, with 1.07 times the error).  From 256 points on, power
+//   where a wavefront takes whole groups 0.5 to 1.05 (shared ones 1.1 to 1.3); two
+//   pols of 256 points, near the memory's rate with one LDS exchange, 0.7 to 1.0;
+//   many long groups 0.8 to 1.0 (power from 2^15 units, four sums from 2^16; half as
+//   many 0.85 to 1.1 and 1.0 to 1.2).
+// - int8 Stokes of 64 points in the longest streams: 0.9 from 2^17 units in groups of
+//   64 (2^16 units, or groups of 32: 1.1 to 1.3).
+static bool vector_pays(const rsd_ctx *d, const ProdPlan &pp, unsigned long long groups, unsigned upg) {
+  const unsigned N = pp.p.Nt;
+  const unsigned long long units = groups * upg;
+  if (N == 1024 && upg == 1) return true;
+  if (d->cfg.Nbps == 16) {
+    if (N == 64 || (N == 256 && d->cfg.Np == 2 && pp.Q == 1)) return true;
+    if (N >= 256 && pp.Q == 1 && (upg < 4 || (groups >= kHybSoloWaves && upg <= kHybSoloUnits))) return true;
+    if (N >= 256 && upg > kHybSoloUnits && units >= (pp.Q == 1 ? 1u << 15 : 1u << 16)) return true;
+  }
+  if (N == 64 && pp.Q != 1 && upg >= 64 && units >= 1u << 17) return true;
+  return (upg == 3 || (upg == 2 && pp.Q == 1)) && groups <= kVecResident;
+}
+
 static void plan_small_h(rsd_ctx *d, ProdPlan &pp) {
-  // int16 power of 64 and 256 points is near the memory's rate on the vector
-  // units (one LDS exchange): 55 and 68 against 69 and 82 us per 256 MiB here
-  pp.h_ok = !pp.bs && rsk::small_h_ok((int)pp.p.Nt, pp.na_buf) &&
-            !(d->cfg.Nbps == 16 && d->cfg.Np == 2 && pp.p.npolout == 1 &&
-              (pp.p.Nt == 64 || pp.p.Nt == 256));
+  pp.h_ok = !pp.bs && rsk::small_h_ok((int)pp.p.Nt, pp.na_buf);
   if (!pp.h_ok) return;
   const unsigned S = 1024u / pp.p.Nt, Nc = d->cfg.Nc;
   const unsigned upg = pp.na_buf / S;          // units per group
+  const unsigned long long groups = (unsigned long long)Nc * pp.Ng;
+  if (vector_pays(d, pp, groups, upg)) {
+    pp.h_ok = 0;
+    return;
+  }
   pp.h_chunk = pp.na_buf;
   pp.h_G = 1;
   pp.h_gpw = 1;
   pp.h_bpc = 1;
   pp.h_waves = 4;
-  const unsigned long long groups = (unsigned long long)Nc * pp.Ng;
-  // Few groups of two or three units: a wavefront takes its units in turn, where
-  // the vector kernel spreads them over a workgroup (55 groups of 3 spectra of
-  // 1024 points, int16 power: 14.3 against 6.8 us, int8 Stokes 10.9 against 9.9;
-  // 1024 groups of int8 12.3 against 14.0, 14.1 against 25.2).  Two units with
-  // four sums are even at 16 groups and better beyond.
-  if ((upg == 3 || (upg == 2 && pp.Q == 1)) && groups < (pp.Q == 1 ? 513u : 512u)) {
-    pp.h_ok = 0;
-    return;
-  }
-  pp.h_solo = groups >= kHybSoloWaves || upg < 4;
+  pp.h_solo = upg < 4 || (groups >= kHybSoloWaves && upg <= kHybSoloUnits);
   if (pp.h_solo) {
     // at most 8 wavefronts per SIMD's two slots, so that the last round is short
     unsigned gpw = (unsigned)(groups / (8ull * kHybSoloWaves));
@@ -469,7 +504,9 @@ static void plan_small_h(rsd_ctx *d, ProdPlan &pp) {
     pp.h_bpc = (pp.Ng + gpw - 1) / gpw;
     return;
   }
-  while (groups * pp.h_G < pp.t_target / 4 && pp.h_chunk % (2 * S) == 0 && pp.h_chunk / (2 * S) >= 4) {
+  while ((groups * pp.h_G < pp.t_target / 4 ||
+          (groups * pp.h_G < pp.t_target && pp.h_chunk > kHybChunkUnits * S)) &&
+         pp.h_chunk % (2 * S) == 0 && pp.h_chunk / (2 * S) >= 4) {
     pp.h_chunk /= 2;
     pp.h_G *= 2;
   }

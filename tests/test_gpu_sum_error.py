@@ -23,6 +23,17 @@ CASES = {
     "8192 two pols": (8192, 128, 1, 1, 2, 8),
     # 256 partial sums of 4 spectra, added by k_reduce
     "1024 one channel": (1024, 1024, 1, 1, 2, 8),
+    # long groups in plenty: whole ones of 8 units a wavefront, shared ones of 16,
+    # 32 and 64; long groups in chunks
+    "64 points, 64 units": (64, 1024, 32, 64, 1, 8),
+    "64 points, 64 units, two pols": (64, 1024, 32, 64, 2, 8),
+    "128 points, 32 units": (128, 256, 64, 32, 2, 8),
+    "128 points int16, 32 units": (128, 256, 64, 32, 2, 16),
+    "256 points, 8 units": (256, 32, 256, 8, 2, 8),
+    "256 points, 64 units": (256, 256, 64, 32, 2, 8),
+    "1024 points, 64 units": (1024, 64, 64, 32, 2, 8),
+    "1024 points int16, 64 units": (1024, 64, 64, 32, 2, 16),
+    "512 points, 256 units": (512, 512, 4, 128, 2, 8),
 }
 
 
