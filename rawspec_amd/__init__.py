@@ -238,13 +238,32 @@ _kept = []
 _made = itertools.count()
 
 
+def _take():
+    try:
+        return _kept.pop()
+    except IndexError:
+        return None
+
+
 def _close_kept():
-    while True:
-        try:
-            sp = _kept.pop()
-        except IndexError:
-            return
+    while (sp := _take()) is not None:
         sp.close()
+
+
+def _keep_newest(sp):
+    # Keeps sp or what was kept, whichever is newer, and closes the rest.
+    # Threads may collect at once: nothing rests on what the list held a step
+    # before, and who leaves two in it takes one up again.
+    while sp is not None:
+        while (old := _take()) is not None:
+            if old._serial > sp._serial:
+                old, sp = sp, old
+            try:
+                old.close()
+            except Exception:
+                pass
+        _kept.append(sp)
+        sp = _take() if len(_kept) > 1 else None
 
 
 def _at_exit():
@@ -464,15 +483,9 @@ class Spectrometer:
 
     def __del__(self):
         try:
-            sp = self
             if self._lent and self.initialized and self._keep:
-                sp = _kept.pop() if _kept else None
-                if sp is not None and sp._serial > self._serial:
-                    sp, newest = self, sp
-                else:
-                    newest = self
-                _kept.append(newest)
-            if sp is not None:
-                sp.close()
+                _keep_newest(self)
+            else:
+                self.close()
         except Exception:
             pass
