@@ -161,8 +161,8 @@ int rawspec_amd_get_held_buffers(rawspec_context *ctx);
  * rawspec_amd_plan() reported only where a chosen plan needs more than the
  * default one).  Writes one line per product ("p<i> N<Nt>
  * <plan>: <best> ms (default <ms> ms, <n> candidates)", milliseconds per
- * buffer of the whole sequence) into report (NUL-terminated; NULL with len 0
- * for none).  Returns 0 on success. */
+ * buffer of the whole sequence; <n>: the different plans timed) into report
+ * (NUL-terminated; NULL with len 0 for none).  Returns 0 on success. */
 int rawspec_amd_autotune(rawspec_context *ctx, const void *d_in, unsigned int per_call,
                          unsigned int rounds, char *report, size_t len);
 

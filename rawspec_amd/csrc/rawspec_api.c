@@ -799,7 +799,7 @@ int rawspec_amd_autotune(rawspec_context *ctx, const void *d_in, unsigned int pe
   g->tuning = 1;
   for (i = 0; i < ctx->No && !rc; i++) {
     const int n = rsd_tune_count(g->dev, (int)i);
-    int k, best = 0;
+    int k, best = 0, timed = 1;
     double t_best, t_dflt;
     char plan[160];
     rc = rsd_tune_apply(g->dev, (int)i, 0);
@@ -812,6 +812,7 @@ int rawspec_amd_autotune(rawspec_context *ctx, const void *d_in, unsigned int pe
       if (a) { rc = 1; break; }
       t = rs_tune_time(ctx, g, d_in, per_call, rounds);
       if (t < 0) { rc = 1; break; }
+      timed++;
       /* a new plan must win clearly: timing noise is a few percent */
       if (t < 0.97 * t_best) { t_best = t; best = k; }
     }
@@ -820,7 +821,7 @@ int rawspec_amd_autotune(rawspec_context *ctx, const void *d_in, unsigned int pe
       int w;
       rsd_tune_describe(g->dev, (int)i, plan, sizeof plan);
       w = snprintf(report + off, len - off, "p%u N%u %s: %.4f ms (default %.4f ms, %d candidates)\n",
-                   i, ctx->Nts[i], plan, t_best * 1e3, t_dflt * 1e3, n);
+                   i, ctx->Nts[i], plan, t_best * 1e3, t_dflt * 1e3, timed);
       if (w > 0) off += (size_t)w < len - off ? (size_t)w : len - off - 1;
     }
   }

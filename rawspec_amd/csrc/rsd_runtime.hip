@@ -1448,7 +1448,8 @@ static std::vector<Tunables> tune_cands(const rsd_ctx *d, const ProdPlan &pp) {
 
 // The launch plan the current tunables produce, for skipping duplicates.
 static std::vector<unsigned long long> plan_key(const ProdPlan &pp) {
-  if (pp.small && pp.h_ok) return {pp.h_chunk, pp.h_gpw, pp.m_chunk};
+  // two chunks in one workgroup of 8 wavefronts have the chunk of the whole group
+  if (pp.small && pp.h_ok) return {pp.h_chunk, pp.h_G, (unsigned long long)pp.h_waves, pp.h_gpw, pp.m_chunk};
   if (pp.small) return {pp.chunk, pp.G, pp.spg, pp.gpw, pp.m_chunk};
   return {pp.fs_chunk, pp.fs_bmax};
 }
@@ -1580,9 +1581,16 @@ int rsd_tune_fit(rsd_ctx *d) {
 
 int rsd_tune_describe(rsd_ctx *d, int i, char *buf, size_t len) {
   const ProdPlan &pp = d->pp[i];
+  if (pp.small && small_on_mfma(d, pp))
+    return snprintf(buf, len, "small matrix-core target %u spg %u mtarget %u (chunk %u)", pp.t_target, pp.t_maxspg,
+                    pp.t_mtarget, pp.m_chunk);
+  if (pp.small && pp.h_ok)
+    return snprintf(buf, len, "small hybrid target %u mtarget %u (chunk %u, %d wavefronts each, %u groups per wavefront)",
+                    pp.t_target, pp.t_mtarget, pp.h_chunk, pp.h_solo ? 1 : pp.h_waves, pp.h_gpw);
   if (pp.small)
-    return snprintf(buf, len, "small target %u spg %u mtarget %u (chunk %u, %u per group, %u groups per workgroup)",
-                    pp.t_target, pp.t_maxspg, pp.t_mtarget, pp.chunk, pp.spg, pp.gpw);
+    return snprintf(buf, len, "small%s target %u spg %u mtarget %u (chunk %u, %u per group, %u groups per workgroup)",
+                    pp.r_ok ? " mixed-radix" : (pp.bs ? " Bluestein" : ""), pp.t_target, pp.t_maxspg, pp.t_mtarget,
+                    pp.chunk, pp.spg, pp.gpw);
   return snprintf(buf, len, "fourstep budget %zu MiB (chunk %u channels, batch %u)", pp.fs_budget >> 20,
                   pp.fs_chunk, pp.fs_bmax);
 }
