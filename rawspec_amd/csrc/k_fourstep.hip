@@ -35,8 +35,7 @@ namespace rsk {
 #define RSK_FS_WG 256
 #endif
 constexpr int kLdsBytes = 160 * 1024;
-template <int NP>
-constexpr int wg_team_np(int n) {
+constexpr int wg_team(int n) {
   // as many teams as RSK_FS_WG asks for, as far as their LDS regions fit
   const int t = n / elems_fs(n);
   const int per_team = n + (n >> 4) + 32;
@@ -45,7 +44,6 @@ constexpr int wg_team_np(int n) {
   while (teams > 1 && (teams * per_team + tw) * 8 > kLdsBytes) teams /= 2;
   return teams * t;
 }
-constexpr int wg_team(int n) { return wg_team_np<2>(n); }
 constexpr int tile_of(int n) { return wg_team(n) / (n / elems_fs(n)); }
 
 // Pass A's workgroup.  From 2048 points a workgroup of 256 threads is two or
@@ -330,11 +328,11 @@ static int go_a_r(int np, const FsArgs &a, unsigned nb, hipStream_t s) {
   if constexpr (N2 == 512 && R1 == 1) {
     if (np != 2 || !a.y24) return 2;
     hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 2, true>), dim3(nb), dim3(WGT), 0, s, a);
-    return hipGetLastError() == hipSuccess ? 0 : 1;
+  } else {
+    if (np == 2 && a.y24) hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 2, true>), dim3(nb), dim3(WGT), 0, s, a);
+    else if (np == 2) hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 2, false>), dim3(nb), dim3(WGT), 0, s, a);
+    else hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 1, false>), dim3(nb), dim3(WGT), 0, s, a);
   }
-  if (np == 2 && a.y24) hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 2, true>), dim3(nb), dim3(WGT), 0, s, a);
-  else if (np == 2) hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 2, false>), dim3(nb), dim3(WGT), 0, s, a);
-  else hipLaunchKernelGGL((k_fs_a<N2, R1, NBPS, 1, false>), dim3(nb), dim3(WGT), 0, s, a);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 

@@ -203,14 +203,17 @@ __global__ __launch_bounds__(256, 2) void k_fs_a_h(FsArgs a) {
 template <int N2, int R1, int NBPS, bool NARROW>
 static int go(int np, const FsArgs &a, unsigned nb, hipStream_t s) {
   const dim3 g(nb), t(256);
+  // narrow only where its loads are (not int16 of two pols up to 128 points)
+  constexpr bool nw2 = NARROW && fs_a_h_load(N2, NBPS, 2, 1) != fs_a_h_load(N2, NBPS, 2, 0);
+  constexpr bool nw1 = NARROW && fs_a_h_load(N2, NBPS, 1, 1) != fs_a_h_load(N2, NBPS, 1, 0);
   if constexpr (N2 < 512) {
     if (np == 2 && a.y24) {
-      hipLaunchKernelGGL((k_fs_a_h<N2, R1, NBPS, 2, true, NARROW>), g, t, 0, s, a);
+      hipLaunchKernelGGL((k_fs_a_h<N2, R1, NBPS, 2, true, nw2>), g, t, 0, s, a);
       return hipGetLastError() == hipSuccess ? 0 : 1;
     }
   }
-  if (np == 2) hipLaunchKernelGGL((k_fs_a_h<N2, R1, NBPS, 2, false, NARROW>), g, t, 0, s, a);
-  else hipLaunchKernelGGL((k_fs_a_h<N2, R1, NBPS, 1, false, NARROW>), g, t, 0, s, a);
+  if (np == 2) hipLaunchKernelGGL((k_fs_a_h<N2, R1, NBPS, 2, false, nw2>), g, t, 0, s, a);
+  else hipLaunchKernelGGL((k_fs_a_h<N2, R1, NBPS, 1, false, nw1>), g, t, 0, s, a);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
