@@ -29,15 +29,25 @@ __global__ __launch_bounds__(256) void k_reduce(ReduceArgs a) {
     // loads (64 partials of 65536 outputs: 42 to 12 us).  Eight running sums,
     // joined pairwise, in a fixed order: one over all partials would round G
     // times in turn.
-    float s[8] = {};
-    for (unsigned ch = 0; ch < a.G; ch += 8) {
-      float v[8];
+    float sum;
+    if (a.G < 8) {
+      sum = p[0];
+      for (unsigned ch = 1; ch < a.G; ++ch) sum += p[ch * step];
+    } else {
+      float s[8] = {};
+      unsigned ch = 0;
+      for (; ch + 8 <= a.G; ch += 8) {
+        float v[8];
 #pragma unroll
-      for (unsigned u = 0; u < 8; ++u) v[u] = ch + u < a.G ? p[(ch + u) * step] : 0.0f;
+        for (int u = 0; u < 8; ++u) v[u] = p[(ch + u) * step];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) s[u] += v[u];
+        for (int u = 0; u < 8; ++u) s[u] += v[u];
+      }
+#pragma unroll
+      for (int u = 0; u < 7; ++u)
+        if (ch + u < a.G) s[u] += p[(ch + u) * step];
+      sum = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
     }
-    const float sum = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
     float *o = a.acc + (((unsigned long long)g * a.Q + q) * a.Nc + c) * a.N + jo;
     const float val = sum * a.scale;
     *o = a.first ? val : (*o + val);

@@ -271,17 +271,17 @@ void k_small(SmallArgs a) {
       if (idx < nout && gg < a.Ng) {
         const float *rp = red + ((go * half) * Q + q) * N + k;
         float sum = rp[0];
-        if (half < 8) {
+        if constexpr (N > 16) {
           for (int s2 = 1; s2 < half; ++s2) sum += rp[s2 * Q * N];
         } else {
-          // many slots: eight running sums, joined pairwise
-          float s[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) s[u] = rp[u * Q * N];
-          for (int s2 = 8; s2 < half; s2 += 8)
-#pragma unroll
-            for (int u = 0; u < 8; ++u) s[u] += rp[(s2 + u) * Q * N];
-          sum = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+          // up to 32 half slots: eight at a time, so that no chain of additions is
+          // longer (from 32 points this took registers and a wavefront per SIMD)
+          for (int s2 = 1; s2 < 8 && s2 < half; ++s2) sum += rp[s2 * Q * N];
+          for (int b = 8; b < half; b += 8) {
+            float t = rp[b * Q * N];
+            for (int s2 = b + 1; s2 < b + 8; ++s2) t += rp[s2 * Q * N];
+            sum += t;
+          }
         }
         if (a.direct) {
           dst[u] = (((unsigned long long)gg * Q + q) * a.Nc + c) * NT + jo;
