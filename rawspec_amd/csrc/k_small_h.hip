@@ -64,8 +64,8 @@ __global__ __launch_bounds__(64 * WAVES, PMODE == 1 ? 3 : 2) void k_small_h(Smal
     const unsigned rest = blockIdx.x - c * (a.Ng * a.G);
     g = rest / a.G;
     chunk = rest - g * a.G;
-    const unsigned cu = a.chunk / S;
-    u0 = g * upg + chunk * cu + wv;
+    const unsigned first = chunk * (a.chunk / S), cu = min(a.chunk / S, upg - first);
+    u0 = g * upg + first + wv;
     ustep = WAVES;
     nu = (unsigned)wv < cu ? (cu - wv + WAVES - 1) / WAVES : 0;
   }
@@ -335,11 +335,12 @@ int launch_small_h(int n, int nbps, int np, int pmode, const SmallArgs &a, unsig
   if (waves != 4 && (waves != 8 || solo)) return 2;
   const unsigned S = 1024u / (unsigned)n;
   // SOLO walks whole groups straight into the integration buffer; otherwise
-  // the chunks are whole units that cover the group
+  // the chunks are whole units that cover the group, the last one perhaps fewer
   if (solo ? (!a.direct || a.G != 1 || a.gpw == 0 || a.bpc == 0 ||
               (unsigned long long)a.bpc * a.gpw < a.Ng ||
               (unsigned long long)nblocks * 4ull < (unsigned long long)a.bpc * a.Nc)
-           : (a.chunk % S != 0 || (unsigned long long)a.chunk * a.G != a.na_buf ||
+           : (a.chunk == 0 || a.chunk % S != 0 || (unsigned long long)a.chunk * a.G < a.na_buf ||
+              (unsigned long long)a.chunk * (a.G - 1) >= a.na_buf ||
               nblocks != (unsigned long long)a.Nc * a.Ng * a.G))
     return 2;
   if (nbps == 8) return go_h_n<8>(n, np, pmode, a, nblocks, solo, waves, s);

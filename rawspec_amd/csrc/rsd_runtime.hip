@@ -504,12 +504,13 @@ static void plan_small_h(rsd_ctx *d, ProdPlan &pp) {
     pp.h_bpc = (pp.Ng + gpw - 1) / gpw;
     return;
   }
-  while ((groups * pp.h_G < pp.t_target / 4 ||
-          (groups * pp.h_G < pp.t_target && pp.h_chunk > kHybChunkUnits * S)) &&
-         pp.h_chunk % (2 * S) == 0 && pp.h_chunk / (2 * S) >= 4) {
-    pp.h_chunk /= 2;
-    pp.h_G *= 2;
+  unsigned cu = upg;                           // units per chunk; the last chunk may have fewer
+  while ((groups * pp.h_G < pp.t_target / 4 || (groups * pp.h_G < pp.t_target && cu > kHybChunkUnits)) &&
+         cu >= 8) {
+    cu = (cu + 1) / 2;
+    pp.h_G = (upg + cu - 1) / cu;
   }
+  pp.h_chunk = cu * S;
   // two chunks fit one workgroup of 8 wavefronts, which saves the partial
   // sums and the launch that adds them (longer serial chains do not pay: 16
   // units by 8 wavefronts 11.0 us, by 16 and k_reduce 9.9)
