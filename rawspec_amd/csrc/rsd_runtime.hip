@@ -396,12 +396,16 @@ static void plan_small(rsd_ctx *d, ProdPlan &pp) {
     unsigned spg = 1;
     while (spg < pp.chunk && spg < kMaxSpg) spg <<= 1;
     // more slots for a long group where that makes too few wavefronts (8
-    // points in dumps of 1024 spectra, 64 MiB: 17 against 47 us; shorter
-    // dumps fill the device as they are and lose by it, 16 against 22)
+    // points in dumps of 1024 spectra, 64 MiB: 17 against 47 us).  With a quarter
+    // of the device's 8192 wavefronts a slot keeps at least 8 spectra (16 points in
+    // dumps of 128, 64 MiB in 2048 wavefronts: 17 us, of 4 spectra 19; in dumps of
+    // 256 24.5, with half as many slots 30), with fewer 4 (16 MiB in dumps of 128:
+    // 7.5, with half as many slots 12)
     const unsigned long long fill = 8192ull * 64 / wg;
-    while (spg < slots && pp.chunk >= 8 * spg &&
-           (unsigned long long)Nc * ((pp.Ng + slots / spg - 1) / (slots / spg)) < fill)
-      spg <<= 1;
+    for (; spg < slots; spg <<= 1) {
+      const unsigned long long wgs = (unsigned long long)Nc * ((pp.Ng + slots / spg - 1) / (slots / spg));
+      if (wgs >= fill || pp.chunk < (wgs < fill / 4 ? 8 : 16) * spg) break;
+    }
     if (spg < slots) {
       pp.spg = spg;
       pp.gpw = slots / spg;
