@@ -113,9 +113,12 @@ void k_small(SmallArgs a) {
       for (int m = 0; m < E; ++m) raw[m] = src[sbase + j + m * T];
     }
     // int8 samples become FP16 pairs; several threads per transform: up to the
-    // first exchange; one thread: dft_pairs
+    // first exchange; one thread: dft_pairs (16 points: dft_bytes)
     constexpr bool kPairs = NBPS == 8 && !BS;
-    if constexpr (kPairs) {
+    if constexpr (kPairs && N == 16) {
+      dft_bytes<0>(raw, v[0], a.isign);
+      if constexpr (NP == 2) dft_bytes<1>(raw, v[NP - 1], a.isign);
+    } else if constexpr (kPairs) {
       h2v x[NP][E];
 #pragma unroll
       for (int m = 0; m < E; ++m) {
