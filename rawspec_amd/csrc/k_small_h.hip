@@ -6,10 +6,11 @@
 // What bounds it: vector instructions.  Per 1024 two-pol int8 samples a
 // wavefront issues about 750 of them (110 unpack, 512 stage 2, 128 Stokes
 // detection) and 32 matrix instructions, which run beside the other
-// wavefront's vector work; the radix 4, 16, 16 vector kernel issues 1383 and
-// exchanges every value through LDS twice.  64 channels x 256 MiB, Stokes, 1024
-// points: 192 + 15 us with its partial sums before, 122 + 7 now; 64 MiB of 256
-// points in dumps of 4: 78 before, 44 now; 128 points, power, 41 and 25.
+// wavefront's vector work (counted over a launch of 16 units a wavefront, with
+// set-up, sums and write-out: 824); the radix 4, 16, 16 vector kernel issues 1383
+// and exchanges every value through LDS twice.  64 channels x 256 MiB, Stokes,
+// 1024 points: 192 + 15 us with its partial sums before, 123 + 7 now; 64 MiB of
+// 256 points in dumps of 4: 78 before, 44 now; 128 points, power, 41 and 25.
 //
 // One wavefront transforms 1024 consecutive samples of a channel at a time
 // (1024 / N spectra, all of one dump group) and loads the next 1024 before

@@ -147,7 +147,7 @@ int launch_fs_a(int nbps, int np, const FsArgs &a, hipStream_t s);
 int fs_a_h_ok(int n1, int n2, int y24);
 int launch_fs_a_h(int nbps, int np, const FsArgs &a, hipStream_t s);
 int launch_fs_b(int np, int pmode, const FsArgs &a, hipStream_t s);
-// The ns runs' sums of a split pass B, in run order, then pass B's own
+// The ns runs' sums of a split pass B, in a fixed order, then pass B's own
 // finish (scale, internal accumulator, shifted output) for a.mode.
 int launch_fs_b_reduce(int pmode, const FsArgs &a, hipStream_t s);
 // The fused small kernel with its first 32 points on the matrix cores (N = 64
